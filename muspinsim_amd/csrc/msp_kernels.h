@@ -85,11 +85,11 @@ hipError_t launch_accumulate(int nslots, int width, const int32_t *ptr, const in
 
 void prof_enable(int on);
 std::string prof_report();
-hipError_t launch_tridiag_lp(int n, int batch, double *H, double *E, double *work, hipStream_t s);
-// Register-resident reduction (matrix in VGPRs, one workgroup of 8 waves per
-// matrix) for 2 <= n <= 64, same outputs as launch_tridiag_lp.
-size_t tridiag_rs_lds_bytes(int n);
-hipError_t launch_tridiag_rs(int n, int batch, double *H, double *E, double *work, hipStream_t s);
+// Householder tridiagonalisation for n <= 1024, kernel chosen by n.
+hipError_t launch_tridiag(int n, int batch, double *H, double *E, double *work, hipStream_t s);
+// Register-resident reduction (matrix in VGPRs, one workgroup per matrix) for
+// n <= 192, same outputs as the panel kernel.
+hipError_t launch_tridiag_rt(int n, int batch, double *H, double *E, double *work, hipStream_t s);
 // U = Q Z on MFMA.  off: rows between a reflector's column and its unit
 // element (1 for the one-stage reduction, 16 for the band stage's panels);
 // nref reflectors; zc: start from the complex Z' = Q2 Z of the two-stage

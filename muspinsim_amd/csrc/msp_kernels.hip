@@ -1127,7 +1127,7 @@ hipError_t launch_eigh_dc(int n, int batch, double *H, double *E, double *U, int
     hipError_t err = hipSuccess;
     if (n <= 1024) {
         ProfScope ps_("k_tridiag", s);
-        err = launch_tridiag_lp(n, batch, H, E, work, s);
+        err = launch_tridiag(n, batch, H, E, work, s);
     } else {
         size_t lds1 = sizeof(cdbl) * 2 * (size_t)n + 16 * sizeof(double);
         err = msp_set_lds((const void *)k_tridiag, lds1);

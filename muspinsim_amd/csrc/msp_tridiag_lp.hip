@@ -24,12 +24,6 @@ constexpr int kPanelRows = 8;   // rows per batched pass of the end-of-panel upd
 #ifndef MSP_TD_RB
 #define MSP_TD_RB 4     // rows per batched pass of the A22 v product (64-lane rows)
 #endif
-#ifndef MSP_TD_ROWS16
-#define MSP_TD_ROWS16 1 // n <= 192: A22 v with one row per 16-lane group
-#endif
-#ifndef MSP_TD_RP
-#define MSP_TD_RP 2     // rows per 16-lane group in one pass of that product
-#endif
 #ifndef MSP_TD_WL
 #define MSP_TD_WL 8     // waves per workgroup above n = 192
 #endif
@@ -48,66 +42,6 @@ constexpr int kPanelRows = 8;   // rows per batched pass of the end-of-panel upd
 
 // reductions across a wave run on DPP lane moves (msp_team.h)
 __device__ inline double wave_sum(double v) { return wave_sum_all(v); }
-
-// Sum over the 16 lanes of each DPP row; every lane of the row gets it.
-__device__ inline double row16_sum(double v)
-{
-    v += dpp_f64<0xB1, 0xF>(v);    // quad_perm [1,0,3,2]
-    v += dpp_f64<0x4E, 0xF>(v);    // quad_perm [2,3,0,1]
-    v += dpp_f64<0x141, 0xF>(v);   // row_half_mirror
-    v += dpp_f64<0x140, 0xF>(v);   // row_mirror
-    return v;
-}
-
-// One pass of the 16-lane-row A22 v product over rows ib + g + 4 W r
-// (r < RP), with the first QA column slots (QA is a compile-time constant so
-// that every load of the pass is issued before the first use).  Slots past a
-// row's diagonal, and rows past n, load A[0][n-1] instead, an element of the
-// strict upper triangle that the kernel zeroes at its start and never writes
-// again, so no loaded value needs a mask.  Every column sum then also takes
-// its diagonal term conj(a_ii) v_i, which the row sum gives back.
-template <int W, int Q16, int QA, int RP>
-__device__ inline void rows16_pass(int n, int k, int ib, int g, int li, const cdbl *A,
-                                   const cdbl *vb, cdbl *pb, cdbl *nxt, cdbl (&colacc)[Q16])
-{
-    cdbl av[RP][QA];
-    cdbl dg[RP];
-#pragma unroll
-    for (int r = 0; r < RP; ++r) {
-        const int i = ib + g + 4 * W * r;
-        const bool rowok = i < n;
-        const int ro = i * n;
-#pragma unroll
-        for (int q = 0; q < QA; ++q) {
-            const int c = k + 1 + li + 16 * q;
-            av[r][q] = A[(rowok && c <= i) ? ro + c : n - 1];
-        }
-        dg[r] = A[rowok ? ro + i : n - 1];
-    }
-#pragma unroll
-    for (int r = 0; r < RP; ++r) {
-        const int i = ib + g + 4 * W * r;
-        const bool rowok = i < n;
-        const cdbl vi = vb[rowok ? i : n - 1];
-        double rr = 0.0, ri = 0.0;
-#pragma unroll
-        for (int q = 0; q < QA; ++q) {
-            const int c = k + 1 + li + 16 * q;
-            const cdbl a = av[r][q];
-            const cdbl vc = vb[(c < n) ? c : n - 1];
-            rr += a.re * vc.re - a.im * vc.im;
-            ri += a.re * vc.im + a.im * vc.re;
-            cfmac(colacc[q], a, vi);
-            if (q == 0 && li == 0 && rowok) nxt[i] = a;   // column k+1
-        }
-        rr = row16_sum(rr);
-        ri = row16_sum(ri);
-        if (li == 0 && rowok) {
-            const cdbl d = dg[r];
-            pb[i] = cmk(rr - (d.re * vi.re + d.im * vi.im), ri - (d.re * vi.im - d.im * vi.re));
-        }
-    }
-}
 
 // Column partials of one step, every thread of the workgroup calling: wave w
 // stores its per-lane sums acc[q] (column c0 + CS q, lanes with `writer`) in
@@ -130,64 +64,6 @@ __device__ inline void store_colpart(int n, int c0, int wave, bool writer, const
             }
         }
     }
-}
-
-#ifndef MSP_TD_QSTEP
-#define MSP_TD_QSTEP 2  // slot-count granularity of the 16-lane-row passes (1 and 4 measured slower)
-#endif
-
-// rows16_pass with the smallest QA = Q16 - MSP_TD_QSTEP m >= qact
-// (qact wave-uniform), so that a pass loads no slot wholly past its rows.
-template <int W, int Q16, int QA, int RP>
-__device__ __forceinline__ void rows16_dispatch(int qact, int n, int k, int ib, int g, int li,
-                                                const cdbl *A, const cdbl *vb, cdbl *pb,
-                                                cdbl *nxt, cdbl (&colacc)[Q16])
-{
-    constexpr int S = MSP_TD_QSTEP;
-    if constexpr (QA > S) {
-        if (qact <= QA - S) {
-            rows16_dispatch<W, Q16, QA - S, RP>(qact, n, k, ib, g, li, A, vb, pb, nxt, colacc);
-            return;
-        }
-    }
-    rows16_pass<W, Q16, QA, RP>(n, k, ib, g, li, A, vb, pb, nxt, colacc);
-}
-
-// A22 v for step k with one matrix row per 16-lane group: wave w takes rows
-// k+1 + 4 W t + 4 w + g (g = lane / 16), a lane the columns k+1 + (lane % 16)
-// + 16 q.  A row sum is a 16-lane DPP reduction shared by the wave's four
-// rows; the column sums conj(a_ic) v_i stay in registers and are combined
-// across the four groups once per step.  pb[i] receives the row sums, nxt[i]
-// the column k+1 (next step's column), cp the waves' column sums.
-template <int W, int Q16>
-__device__ inline void matvec_rows16(int n, int k, int wave, int lane, const cdbl *A, const cdbl *vb,
-                                     cdbl *pb, cdbl *nxt, cdbl *cp)
-{
-    static_assert(Q16 == 4 || Q16 == 8 || Q16 == 12, "16-lane rows cover n <= 192");
-    const int g = lane >> 4, li = lane & 15;
-    cdbl colacc[Q16];
-#pragma unroll
-    for (int q = 0; q < Q16; ++q) colacc[q] = cmk(0.0, 0.0);
-    constexpr int RP = MSP_TD_RP;
-    for (int ib = k + 1 + 4 * wave; ib < n; ib += 4 * W * RP) {
-        const int ilast0 = ib + 4 * W * (RP - 1) + 3;
-        const int ilast = (ilast0 < n) ? ilast0 : n - 1;
-        const int qact = ((ilast - (k + 1)) >> 4) + 1;          // wave-uniform, <= Q16
-        rows16_dispatch<W, Q16, Q16, RP>(qact, n, k, ib, g, li, A, vb, pb, nxt, colacc);
-    }
-    const int qstep = ((n - 1 - (k + 1)) >> 4) + 1;
-#pragma unroll
-    for (int q = 0; q < Q16; ++q) {
-        if (q < qstep) {
-            cdbl t = colacc[q];
-            t.re += __shfl_xor(t.re, 16, 64);
-            t.im += __shfl_xor(t.im, 16, 64);
-            t.re += __shfl_xor(t.re, 32, 64);
-            t.im += __shfl_xor(t.im, 32, 64);
-            colacc[q] = t;
-        }
-    }
-    store_colpart<W, Q16, 16>(n, k + 1 + li, wave, g == 0, colacc, cp);
 }
 
 // End-of-panel rank-2k update with lanes owning columns: for each 64-column
@@ -369,7 +245,7 @@ __device__ __forceinline__ int a22v_rows(int n, int k, int i0, int lane, const c
     return RB * W;
 }
 
-template <int W, int NB, int QMAX, int RB, int Q16, bool GP>
+template <int W, int NB, int QMAX, int RB, bool GP>
 __global__ void __launch_bounds__(64 * W) k_tridiag_lp(int n, double *H, double *E, double *work)
 {
     static_assert(W == 4 || W == 8, "4 or 8 waves per matrix");
@@ -398,10 +274,6 @@ __global__ void __launch_bounds__(64 * W) k_tridiag_lp(int n, double *H, double 
     cdbl *stage = (cdbl *)(red + 2 * W);             // GP: 64 MSP_TD_SPL per wave
 
     cdbl *col = colA, *nxt = colB;
-    // A[0][n-1] (strict upper triangle, never written below) is the zero that
-    // the 16-lane-row A22 v passes load in place of elements past a row's
-    // diagonal; the first barrier below publishes it
-    if (Q16 > 0 && tid == 0) A[n - 1] = cmk(0.0, 0.0);
     for (int i = tid; i < n; i += kThreads) col[i] = A[(size_t)i * n];
     for (int k0 = 0; k0 < n - 1; k0 += NB) {
         const int nbk = (n - 1 - k0 < NB) ? n - 1 - k0 : NB;
@@ -481,21 +353,17 @@ __global__ void __launch_bounds__(64 * W) k_tridiag_lp(int n, double *H, double 
                     if (lane == 0) y[l] = cmk(sr, si);
                 }
                 // (d) A22 v over the lower triangle of rows/cols k+1..n-1
-                if constexpr (Q16 > 0) {
-                    matvec_rows16<W, Q16>(n, k, wave, lane, A, vb, pb, nxt, cp);
-                } else {
-                    cdbl colacc[QMAX];
-    #pragma unroll
-                    for (int q = 0; q < QMAX; ++q) colacc[q] = cmk(0.0, 0.0);
-                    // RB rows per pass (i, i+W, ... of this wave): every load of
-                    // the pass is issued first, from clamped addresses with the
-                    // value masked, so no branch separates the loads
-                    // (slots past a pass's longest row hold c > i for every
-                    // lane and row: neither loaded nor used)
-                    for (int i0 = k + 1 + wave; i0 < n;)
-                        i0 += a22v_rows<W, QMAX, RB>(n, k, i0, lane, A, vb, pb, nxt, colacc);
-                    store_colpart<W, QMAX, 64>(n, k + 1 + lane, wave, true, colacc, cp);
-                }
+                cdbl colacc[QMAX];
+#pragma unroll
+                for (int q = 0; q < QMAX; ++q) colacc[q] = cmk(0.0, 0.0);
+                // RB rows per pass (i, i+W, ... of this wave): every load of
+                // the pass is issued first, from clamped addresses with the
+                // value masked, so no branch separates the loads
+                // (slots past a pass's longest row hold c > i for every
+                // lane and row: neither loaded nor used)
+                for (int i0 = k + 1 + wave; i0 < n;)
+                    i0 += a22v_rows<W, QMAX, RB>(n, k, i0, lane, A, vb, pb, nxt, colacc);
+                store_colpart<W, QMAX, 64>(n, k + 1 + lane, wave, true, colacc, cp);
                 __syncthreads();
                 // (e) p = tau (A22 v - Vp y1 - Wp y2), and p^H v
                 double pre = 0.0, pim = 0.0;
@@ -567,31 +435,27 @@ size_t lp_lds(int n)
            16 * sizeof(double);
 }
 
-template <int W, int NB, int QMAX, int RB, int Q16, bool GP = false>
+template <int W, int NB, int QMAX, int RB, bool GP = false>
 hipError_t lp_launch(int n, int batch, double *H, double *E, double *work, hipStream_t s)
 {
     size_t lds = lp_lds<W, NB, GP>(n);
-    hipError_t err = msp_set_lds((const void *)k_tridiag_lp<W, NB, QMAX, RB, Q16, GP>, lds);
+    hipError_t err = msp_set_lds((const void *)k_tridiag_lp<W, NB, QMAX, RB, GP>, lds);
     if (err != hipSuccess) return err;
-    hipLaunchKernelGGL((k_tridiag_lp<W, NB, QMAX, RB, Q16, GP>), dim3(batch), dim3(64 * W), lds, s, n,
+    hipLaunchKernelGGL((k_tridiag_lp<W, NB, QMAX, RB, GP>), dim3(batch), dim3(64 * W), lds, s, n,
                        H, E, work);
     return hipGetLastError();
 }
 
 }  // namespace
 
-// Lower-triangle panel kernel for n <= 1024 (panels in the workspace above
-// n = 512); returns hipErrorNotSupported above.
-hipError_t launch_tridiag_lp(int n, int batch, double *H, double *E, double *work, hipStream_t s)
+// Householder tridiagonalisation for n <= 1024 (hipErrorNotSupported above):
+// the register-resident kernel where the matrix fits one CU's registers, the
+// lower-triangle panel kernel above (panels in the workspace from n = 513 on).
+hipError_t launch_tridiag(int n, int batch, double *H, double *E, double *work, hipStream_t s)
 {
-    // n <= 64: the register-resident kernel (msp_tridiag_rs.hip) is faster
-    if (n >= 2 && n <= 64) return launch_tridiag_rs(n, batch, H, E, work, s);
-    if (n <= 64) return lp_launch<4, 8, 1, MSP_TD_RB, MSP_TD_ROWS16 ? 4 : 0>(n, batch, H, E, work, s);
-    if (n <= 128) return lp_launch<4, 8, 2, MSP_TD_RB, MSP_TD_ROWS16 ? 8 : 0>(n, batch, H, E, work, s);
-    if (n <= 192) return lp_launch<4, 8, 3, MSP_TD_RB, MSP_TD_ROWS16 ? 12 : 0>(n, batch, H, E, work, s);
-    // above n = 192 one workgroup fills a CU's LDS: 8 waves put two on each SIMD
-    if (n <= 256) return lp_launch<MSP_TD_WL, 8, 4, 4, 0>(n, batch, H, E, work, s);
-    if (n <= 512) return lp_launch<MSP_TD_WL, 4, 8, 4, 0>(n, batch, H, E, work, s);
-    if (n <= 1024) return lp_launch<MSP_TD_WL, MSP_TD_NBL, 16, MSP_TD_RB1024, 0, true>(n, batch, H, E, work, s);
+    if (n <= 192) return launch_tridiag_rt(n, batch, H, E, work, s);
+    if (n <= 256) return lp_launch<MSP_TD_WL, 8, 4, 4>(n, batch, H, E, work, s);
+    if (n <= 512) return lp_launch<MSP_TD_WL, 4, 8, 4>(n, batch, H, E, work, s);
+    if (n <= 1024) return lp_launch<MSP_TD_WL, MSP_TD_NBL, 16, MSP_TD_RB1024, true>(n, batch, H, E, work, s);
     return hipErrorNotSupported;
 }

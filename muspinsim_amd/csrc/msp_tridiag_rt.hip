@@ -1,0 +1,424 @@
+// Householder tridiagonalisation with the matrix resident in the registers of
+// one CU (gfx950, n <= 192).  Same reduction and outputs as the panel kernel
+// (msp_tridiag_lp.hip): reflectors v with v_{k+1} = 1, tails below the
+// subdiagonal of the row-major matrix, d to E, e and tau to the workspace.
+//
+// Layout: rows go in strips of 4 W (W waves); lane l of wave w holds row
+// 4 w + l / 16 of every strip and column l % 16 of every 16-column block up to
+// the strip's diagonal region, which is held whole.  Every wave has the same
+// static code and the same share of the live matrix at every step; row sums
+// stay in one wave, column sums cross the W waves once per step through LDS.
+//
+// Column step k:
+//   1. wave 0 brings column k up to date and forms its reflector, the others
+//      meanwhile apply the previous step's rank-2 update to the live blocks;
+//   2. A22 x' over the live blocks, row sums and (by Hermitian symmetry)
+//      column sums; x' is the column with its first entry replaced by
+//      alpha - beta, so v = x' / (alpha - beta); column k + 1 goes to LDS;
+//   3. per row: the sums are added and v and
+//      w = tau A22 v - (|tau|^2 / 2)(v^H A22 v) v, whose scalar is real, formed.
+// Three workgroup barriers per column; global memory is read once.
+//
+// What bounds it: at n = 192 about 480 vector instructions per wave and column
+// (300 of them FP64 FMAs, 190 of those the live lower triangle's) keep the
+// SIMDs half busy; the rest is the reflector's serial chain, the barriers and
+// LDS (37 % busy).  At one 8-wave workgroup per CU nothing covers the barriers;
+// below n = 128 two to sixteen workgroups share a CU.
+// The panel kernel re-reads the trailing triangle once per column (at n = 192
+// 5.2 TB/s past L2); here the matrix is read once.  ms per 4096 matrices, panel
+// kernel (below n = 65: registers in 64-column slots) against this one:
+//   n = 192 18.6 / 10.3, 144 10.7 / 6.6, 128 8.3 / 3.2, 108 6.2 / 2.5,
+//   96 5.1 / 1.7, 72 3.3 / 1.1, 64 2.25 / 0.74, 48 1.82 / 0.37, 32 0.91 / 0.19,
+//   16 0.47 / 0.06; one matrix: n = 192 1.88 / 0.62, 64 0.18 / 0.11.
+// Measured and not taken: 16 x 16 tiles in MFMA accumulators dealt to the waves
+// with the rank-2 update on MFMA (n = 192 14.6 ms: FP64 MFMA and FP64 VALU
+// share one pipe, so the products delay the other waves' serial chains, and a
+// branch per tile costs register copies); row sums by DPP halving instead of
+// through LDS (10.5 ms).
+#include <hip/hip_runtime.h>
+
+#include <utility>
+
+#include "msp_kernels.h"
+#include "msp_tridiag.h"
+
+namespace {
+
+__device__ inline void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+__device__ inline void swap32(double &x, double &y)
+{
+    const unsigned long long a = (unsigned long long)__double_as_longlong(x);
+    const unsigned long long b = (unsigned long long)__double_as_longlong(y);
+    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)a, (unsigned)b, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(a >> 32), (unsigned)(b >> 32), false, false);
+    x = __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0]));
+    y = __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
+}
+__device__ inline void swap16(double &x, double &y)
+{
+    const unsigned long long a = (unsigned long long)__double_as_longlong(x);
+    const unsigned long long b = (unsigned long long)__double_as_longlong(y);
+    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)a, (unsigned)b, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(a >> 32), (unsigned)(b >> 32), false, false);
+    x = __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0]));
+    y = __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
+}
+
+// Square root and its reciprocal of t > 0: hardware estimate, two coupled
+// Newton steps, and a last correction of the root.
+__device__ inline void sqrt_recip(double t, double &root, double &rec)
+{
+    const double y = __builtin_amdgcn_rsq(t);
+    double gg = t * y, h = 0.5 * y;
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+        const double r = fma(-gg, h, 0.5);
+        gg = fma(gg, r, gg);
+        h = fma(h, r, h);
+    }
+    root = fma(fma(-gg, gg, t), h, gg);
+    rec = 2.0 * h;
+}
+
+__device__ inline double readlane_f64(double v, int l)
+{
+    const long long x = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)(x & 0xffffffffll), l);
+    const int hi = __builtin_amdgcn_readlane((int)(x >> 32), l);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// Value of lane L of this lane's row of 16 lanes.
+template <int L>
+__device__ inline double row_bcast(double v)
+{
+    return __longlong_as_double(
+        __builtin_amdgcn_update_dpp(0ll, __double_as_longlong(v), 0x150 + L, 0xF, 0xF, true));
+}
+// o[a] = x of lane FIRST + STEP a of each row of 16 lanes
+template <int FIRST, int STEP, int NS, int... I>
+__device__ inline void spread(cdbl x, cdbl (&o)[NS], std::integer_sequence<int, I...>)
+{
+    ((o[I] = cmk(row_bcast<FIRST + STEP * I>(x.re), row_bcast<FIRST + STEP * I>(x.im))), ...);
+}
+
+// W: waves, NS: strips of 4 W rows (n <= 4 W NS), OCC: waves per SIMD asked for.
+template <int W, int NS>
+struct RtShape {
+    static constexpr int SR = 4 * W;                       // rows per strip
+    static constexpr int NR = SR * NS;
+    // first and last column block of strip a's diagonal region
+    static constexpr int j0(int a) { return a * W / 4; }
+    static constexpr int dl(int a) { return W >= 4 ? j0(a) + W / 4 - 1 : j0(a); }
+    static constexpr int slot(int a, int J)
+    {
+        int s = 0;
+        for (int b = 0; b < a; ++b) s += dl(b) + 1;
+        return s + J;
+    }
+    static constexpr int NJ = dl(NS - 1) + 1;
+    static constexpr int NSLOT = slot(NS, 0);
+    static constexpr int NC = (NR + 63) / 64;              // entries per lane of a vector
+    static constexpr int NP = 64 * NC;
+    // LDS: x', column k + 1, v and w, column sums per wave, row sums per lane,
+    // scale, tau scale, -|tau scale|^2 / 2, and a share of v^H A22 v per wave
+    static constexpr int CDBL = 4 * NP + W * NP + 64 * W * NS + 3;
+    static constexpr size_t LDS = sizeof(cdbl) * CDBL + sizeof(double) * ((W + 1) & ~1);
+};
+
+template <int W, int NS, int OCC>
+__global__ void __launch_bounds__(64 * W, OCC) k_tridiag_rt(int n, double *H, double *E, double *work)
+{
+    using T = RtShape<W, NS>;
+    constexpr int SR = T::SR, NJ = T::NJ, NC = T::NC, NP = T::NP;
+    static_assert(NS <= 8, "two lanes per row of a wave");
+    extern __shared__ __align__(16) unsigned char smem[];
+    cdbl *col = (cdbl *)smem;                  // x': zero up to row k
+    cdbl *cn = col + NP;                       // column k + 1 before step k's update
+    cdbl *V = cn + NP, *Wv = V + NP;           // v and w of the pending update
+    cdbl *P = Wv + NP;                         // column sums per wave
+    cdbl *R = P + W * NP;                      // row sums per lane: [wave][strip][g][c]
+    cdbl *scal = R + 64 * W * NS;              // scale, tau scale, (-|tau scale|^2 / 2, -)
+    double *dot = (double *)(scal + 3);
+
+    const int b0 = blockIdx.x;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, c = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    cdbl *A = (cdbl *)H + (size_t)b0 * n * n;
+    double *base = work + (size_t)b0 * dc_work_doubles(n);
+    double *e;
+    cdbl *tau;
+    dc_carve(n, base, &e, &tau);
+    double *d = E + (size_t)b0 * n;
+
+    cdbl M[T::NSLOT];
+#pragma unroll
+    for (int a = 0; a < NS; ++a)
+#pragma unroll
+        for (int J = 0; J <= T::dl(a); ++J) {
+            const int row = SR * a + 4 * wave + g, cc = 16 * J + c;
+            cdbl x = cmk(0.0, 0.0);
+            if (row < n && cc < n) {
+                x = (row >= cc) ? A[(size_t)row * n + cc] : A[(size_t)cc * n + row];
+                if (row < cc) x.im = -x.im;
+                if (row == cc) x.im = 0.0;
+            }
+            M[T::slot(a, J)] = x;
+        }
+    for (int i = tid; i < NP; i += 64 * W) {
+        V[i] = Wv[i] = cmk(0.0, 0.0);
+        cn[i] = (i < n) ? A[(size_t)i * n] : cmk(0.0, 0.0);
+    }
+    for (int i = tid; i < W * NP + 64 * W * NS; i += 64 * W) P[i] = cmk(0.0, 0.0);
+    // LDS places of this lane: its rows and columns, its share of the sums
+    const cdbl *vrp = V + NP * (c & 1) + SR * min(c >> 1, NS - 1) + 4 * wave + g;
+    const cdbl *xrp = col + SR * min(c, NS - 1) + 4 * wave + g;
+    double *Pw = (double *)(P + wave * NP + 16 * (g >> 1) + c) + (g & 1);
+    cdbl *Rw = R + 64 * wave * NS + lane;
+    // stage 3: lane halves share a row, half h adds the column sums of its
+    // waves and the row sums of its eight columns, from a different column in
+    // each lane so that the lanes read different banks
+    const int h = lane >> 5, rr = lane & 31;
+    const int i3 = SR * (rr >> 2) + 4 * wave + (rr & 3);
+    const cdbl *Rs = R + 64 * wave * NS + 16 * min(rr, 4 * NS - 1);
+    const int u3 = rr + 8 * h;
+    __syncthreads();
+
+    for (int k = 0;; ++k) {
+        const int jp1 = (k + 1) >> 5;          // pairs of column blocks before it are done
+        // (1) wave 0: column k with the pending update and its reflector
+        if (wave == 0) {
+            __builtin_amdgcn_s_setprio(2);
+            cdbl x[NC];
+            const double vkr = V[k].re, vki = V[k].im, wkr = Wv[k].re, wki = Wv[k].im;
+#pragma unroll
+            for (int t = 0; t < NC; ++t) {
+                const int i = 64 * t + lane;
+                const double vr = V[i].re, vi = V[i].im, wr = Wv[i].re, wi = Wv[i].im;
+                x[t] = cn[i];
+                x[t].re = fma(-vr, wkr, x[t].re);
+                x[t].im = fma(-vi, wkr, x[t].im);
+                x[t].re = fma(-vi, wki, x[t].re);
+                x[t].im = fma(vr, wki, x[t].im);
+                x[t].re = fma(-wr, vkr, x[t].re);
+                x[t].im = fma(-wi, vkr, x[t].im);
+                x[t].re = fma(-wi, vki, x[t].re);
+                x[t].im = fma(wr, vki, x[t].im);
+            }
+            double part = 0.0, dk = 0.0;
+            cdbl alpha = cmk(0.0, 0.0);
+#pragma unroll
+            for (int t = 0; t < NC; ++t) {
+                const int i = 64 * t + lane;
+                part += (i > k + 1) ? cabs2(x[t]) : 0.0;
+                dk = (i == k) ? x[t].re : dk;
+                const cdbl a = cmk(readlane_f64(x[t].re, (k + 1) & 63), readlane_f64(x[t].im, (k + 1) & 63));
+                if (((k + 1) >> 6) == t) alpha = a;
+            }
+            if (lane == (k & 63)) d[k] = dk;
+            if (k == n - 1) break;
+            const double xn2 = wave_sum_all(part);
+            cdbl tk = cmk(0.0, 0.0), scale = tk, xh = tk;
+            double beta = alpha.re;
+            if (!(xn2 == 0.0 && alpha.im == 0.0)) {
+                double nrm, rb;
+                sqrt_recip(fma(alpha.re, alpha.re, fma(alpha.im, alpha.im, xn2)), nrm, rb);
+                beta = alpha.re >= 0.0 ? -nrm : nrm;
+                rb = alpha.re >= 0.0 ? -rb : rb;
+                // tau = (beta - alpha)/beta, 1/(alpha - beta) = (1/beta)/d with
+                // d = alpha/beta - 1, 1 <= |d| <= 2
+                tk = cmk((beta - alpha.re) * rb, -alpha.im * rb);
+                const double dr = fma(alpha.re, rb, -1.0), di = alpha.im * rb;
+                const double rd = rb * msp_recip(fma(dr, dr, di * di));
+                scale = cmk(dr * rd, -di * rd);
+                xh = cmk(alpha.re - beta, alpha.im);
+            }
+#pragma unroll
+            for (int t = 0; t < NC; ++t) {
+                const int i = 64 * t + lane;
+                col[i] = (i > k + 1) ? x[t] : (i == k + 1 ? xh : cmk(0.0, 0.0));
+            }
+            if (lane == 0) {
+                const cdbl u = cmul(tk, scale);
+                scal[0] = scale;
+                scal[1] = u;
+                scal[2] = cmk(-0.5 * cabs2(u), 0.0);
+                e[k] = beta;
+                tau[k] = tk;
+            }
+            __builtin_amdgcn_s_setprio(0);
+            lds_barrier();
+        } else if (k == n - 1) {
+            break;
+        }
+
+        // pending update A22 -= v w^H + w v^H of the live blocks
+        if (k > 0) {
+            // lane c of a row of 16 reads v (c even) or w (c odd) of strip c / 2
+            cdbl vr[NS], wr[NS];
+            const cdbl ro = *vrp;
+            spread<0, 2>(ro, vr, std::make_integer_sequence<int, NS>());
+            spread<1, 2>(ro, wr, std::make_integer_sequence<int, NS>());
+#pragma unroll
+            for (int jp = 0; jp < (NJ + 1) / 2; ++jp) {
+                if (jp < jp1) continue;
+#pragma unroll
+                for (int J = 2 * jp; J < 2 * jp + 2 && J < NJ; ++J) {
+                    const cdbl vj = V[16 * J + c], wj = Wv[16 * J + c];
+#pragma unroll
+                    for (int a = 0; a < NS; ++a) {
+                        if (J > T::dl(a)) continue;
+                        cdbl &m = M[T::slot(a, J)];
+                        m.re = fma(-vr[a].re, wj.re, m.re);
+                        m.im = fma(-vr[a].im, wj.re, m.im);
+                        m.re = fma(-vr[a].im, wj.im, m.re);
+                        m.im = fma(vr[a].re, wj.im, m.im);
+                        m.re = fma(-wr[a].re, vj.re, m.re);
+                        m.im = fma(-wr[a].im, vj.re, m.im);
+                        m.re = fma(-wr[a].im, vj.im, m.re);
+                        m.im = fma(wr[a].re, vj.im, m.im);
+                    }
+                }
+            }
+        }
+        if (wave != 0) lds_barrier();
+
+        // (2) A22 x' over the live blocks
+        {
+            cdbl xr[NS], rs[NS];
+            double dacc = 0.0;
+#pragma unroll
+            for (int a = 0; a < NS; ++a) rs[a] = cmk(0.0, 0.0);
+            spread<0, 1>(*xrp, xr, std::make_integer_sequence<int, NS>());
+#pragma unroll
+            for (int jp = 0; jp < (NJ + 1) / 2; ++jp) {
+                if (jp < jp1) continue;
+                cdbl cs[2];
+                cs[0] = cs[1] = cmk(0.0, 0.0);
+#pragma unroll
+                for (int J = 2 * jp; J < 2 * jp + 2 && J < NJ; ++J) {
+                    const cdbl xc = col[16 * J + c];
+#pragma unroll
+                    for (int a = 0; a < NS; ++a) {
+                        if (J > T::dl(a)) continue;
+                        const cdbl m = M[T::slot(a, J)];
+                        if (J < T::j0(a)) cfmac(cs[J & 1], m, xr[a]);
+                        // v^H A22 v counts the blocks left of the diagonal region twice
+                        if (J == T::j0(a)) dacc = fma(xr[a].re, rs[a].re, fma(xr[a].im, rs[a].im, dacc));
+                        cfma(rs[a], m, xc);
+                    }
+                }
+                // column k + 1 for the next step
+#pragma unroll
+                for (int J = 2 * jp; J < 2 * jp + 2 && J < NJ; ++J) {
+                    if (J != ((k + 1) >> 4)) continue;
+                    if (c == ((k + 1) & 15)) {
+#pragma unroll
+                        for (int a = 0; a < NS; ++a)
+                            if (J <= T::dl(a)) cn[SR * a + 4 * wave + g] = M[T::slot(a, J)];
+                    }
+                }
+                if (2 * jp < T::j0(NS - 1)) {
+                    swap32(cs[0].re, cs[1].re);
+                    swap32(cs[0].im, cs[1].im);
+                    double s = cs[0].re + cs[1].re, t = cs[0].im + cs[1].im;
+                    swap16(s, t);
+                    Pw[64 * jp] = s + t;
+                }
+            }
+#pragma unroll
+            for (int a = 0; a < NS; ++a) dacc = fma(xr[a].re, rs[a].re, fma(xr[a].im, rs[a].im, dacc));
+            // row sums of the live strips, left to stage 3 (this wave's rows)
+            if (k + 1 < SR * (NS / 2)) {
+#pragma unroll
+                for (int a = 0; a < NS / 2; ++a) Rw[64 * a] = rs[a];
+            }
+#pragma unroll
+            for (int a = NS / 2; a < NS; ++a) Rw[64 * a] = rs[a];
+            dacc = wave_sum_all(dacc);
+            if (lane == 0) dot[wave] = dacc;
+        }
+        lds_barrier();
+
+        // (3) v and w of this wave's rows
+        if (SR * (NS - 1) + 4 * wave + 3 >= k) {
+            const bool in = rr < 4 * NS;
+            const int i = in ? i3 : 0;
+            cdbl y = Rs[u3 & 15];
+#pragma unroll
+            for (int u = 1; u < 8; ++u) y = cadd(y, Rs[(u + u3) & 15]);
+            const cdbl xi = col[i], scale = scal[0], u = scal[1];
+            const double mh = scal[2].re;
+            double rho = 0.0;
+#pragma unroll
+            for (int w = 0; w < W; ++w) rho += dot[w];
+#pragma unroll
+            for (int w = 0; w < (W + 1) / 2; ++w)
+                if (W > 1 || h == 0) y = cadd(y, P[(w + h * (W / 2)) * NP + i]);
+            double t = y.re;
+            swap32(y.re, t);
+            y.re += t;
+            t = y.im;
+            swap32(y.im, t);
+            y.im += t;
+            const bool act = u.re != 0.0 || u.im != 0.0;
+            const cdbl v = (i == k + 1) ? cmk(act ? 1.0 : 0.0, 0.0) : cmul(xi, scale);
+            const cdbl p = cmul(u, y);
+            const double c0 = mh * rho;
+            cdbl o = h ? cmk(fma(c0, v.re, p.re), fma(c0, v.im, p.im)) : v;
+            if (!(i > k && i < n)) o = cmk(0.0, 0.0);
+            if (in) V[NP * h + i] = o;
+            if (in && h == 0 && i >= k + 2 && i < n) A[(size_t)i * n + k] = v;
+        }
+        lds_barrier();
+    }
+}
+
+template <int W, int NS, int OCC>
+hipError_t rt_launch(int n, int batch, double *H, double *E, double *work, hipStream_t s)
+{
+    const size_t lds = RtShape<W, NS>::LDS;
+    hipError_t err = msp_set_lds((const void *)k_tridiag_rt<W, NS, OCC>, lds);
+    if (err != hipSuccess) return err;
+    hipLaunchKernelGGL((k_tridiag_rt<W, NS, OCC>), dim3(batch), dim3(64 * W), lds, s, n, H, E, work);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+// Waves and strips by n: one wave per 16 rows of small matrices, so that many
+// matrices share a CU, four waves where two or more workgroups still fit its
+// registers (n <= 128), eight above.  Strips of 4 W rows cover n closely: a
+// strip too many costs 10 to 20 %.
+// Up to 512 matrices run at most two to a CU and take the form with the
+// shortest column step; more take the form that holds more matrices per CU.
+// ms for 256 / 4096 matrices: n = 48 four waves 0.078 / 0.44, two 0.095 /
+// 0.37; n = 96 at two workgroups per CU 0.205 / 1.93, at three (four registers
+// spilled) 0.230 / 1.71; n = 32 two waves 0.051 / 0.19, one 0.058 / 0.19;
+// n = 128 four waves 0.32 / 3.1, eight 0.31 / 4.9.
+hipError_t launch_tridiag_rt(int n, int batch, double *H, double *E, double *work, hipStream_t s)
+{
+    const bool many = batch > 512;
+    if (n <= 12) return rt_launch<1, 3, 4>(n, batch, H, E, work, s);
+    if (n <= 16) return rt_launch<1, 4, 4>(n, batch, H, E, work, s);
+    if (n <= 24) return rt_launch<2, 3, 4>(n, batch, H, E, work, s);
+    if (n <= 32) return rt_launch<2, 4, 4>(n, batch, H, E, work, s);
+    if (n <= 48 && many) return rt_launch<2, 6, 4>(n, batch, H, E, work, s);
+    if (n <= 48) return rt_launch<4, 3, 4>(n, batch, H, E, work, s);
+    if (n <= 64) return rt_launch<4, 4, 4>(n, batch, H, E, work, s);
+    if (n <= 80) return rt_launch<4, 5, 3>(n, batch, H, E, work, s);
+    if (n <= 96 && many) return rt_launch<4, 6, 3>(n, batch, H, E, work, s);
+    if (n <= 96) return rt_launch<4, 6, 2>(n, batch, H, E, work, s);
+    if (n <= 112) return rt_launch<4, 7, 2>(n, batch, H, E, work, s);
+    if (n <= 128) return rt_launch<4, 8, 2>(n, batch, H, E, work, s);
+    if (n <= 160) return rt_launch<8, 5, 2>(n, batch, H, E, work, s);
+    if (n <= 192) return rt_launch<8, 6, 2>(n, batch, H, E, work, s);
+    return hipErrorNotSupported;
+}

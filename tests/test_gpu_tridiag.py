@@ -1,0 +1,62 @@
+"""Register-resident Householder tridiagonalisation (through msp_eigh's divide
+and conquer) at the edges of its strips and column blocks, on structured
+matrices and on both sides of its batch rule."""
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def eng(gpu_lib):
+    from muspinsim_amd.engine import SpinEngine
+    return SpinEngine("cuda:0")
+
+
+def _herm(rng, n):
+    X = rng.normal(size=(n, n)) + 1j * rng.normal(size=(n, n))
+    return (X + X.conj().T) / 2
+
+
+def _check(eng, Hs):
+    """Backward error of order n eps ||H|| and orthonormal eigenvectors; the
+    strict upper triangle, which the solver must not read, is NaN."""
+    from muspinsim_amd import _native as N
+    n = Hs.shape[1]
+    low = Hs.copy()
+    low[:, np.triu_indices(n, 1)[0], np.triu_indices(n, 1)[1]] = np.nan
+    E, U, info = eng.eigh(torch.as_tensor(low).cuda(), method=N.MSP_EIGH_DC)
+    E, U = E.cpu().numpy(), U.cpu().numpy()
+    assert np.all(info.cpu().numpy() == 0)
+    nrm = np.maximum(np.abs(E).max(1), 1e-300)
+    assert np.all(np.abs(E - np.linalg.eigvalsh(Hs)).max(1) <= 1e-14 * n * nrm)
+    assert np.all(np.abs(Hs @ U - U * E[:, None, :]).max((1, 2)) <= 1e-14 * n * nrm)
+    UU = np.conj(np.swapaxes(U, 1, 2)) @ U
+    assert np.abs(UU - np.eye(n)).max() <= 1e-14 * max(n, 10)
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 11, 12, 13, 15, 16, 17, 24, 25, 31, 32, 33, 48, 49, 64, 65,
+                               80, 81, 95, 96, 97, 108, 112, 113, 127, 128, 129, 160, 161, 191,
+                               192, 193])
+def test_structured(eng, n):
+    rng = np.random.default_rng(n)
+    tri = np.diag(rng.normal(size=n)) + 0j
+    i = np.arange(n - 1)
+    tri[i + 1, i] = rng.normal(size=n - 1) + 1j * rng.normal(size=n - 1)
+    tri[i, i + 1] = np.conj(tri[i + 1, i])
+    v = rng.normal(size=n) + 1j * rng.normal(size=n)
+    half = np.zeros((n, n), dtype=complex)     # two uncoupled blocks: a zero column on the way
+    m = n // 2
+    half[:m, :m], half[m:, m:] = _herm(rng, m), _herm(rng, n - m)
+    _check(eng, np.array([_herm(rng, n), 1e6 * _herm(rng, n), np.zeros((n, n)) + 0j,
+                          np.diag(rng.normal(size=n)) + 0j, tri, np.outer(v, v.conj()),
+                          _herm(rng, n).real + 0j, half]))
+
+
+@pytest.mark.parametrize("n", [40, 90])
+@pytest.mark.parametrize("batch", [512, 513])
+def test_batch_rule(eng, n, batch):
+    rng = np.random.default_rng(n + batch)
+    _check(eng, np.array([_herm(rng, n) for _ in range(batch)]))
