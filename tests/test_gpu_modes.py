@@ -1,0 +1,65 @@
+"""Mode decomposition of general complex matrices (msp_lindblad_modes without
+eigenvectors) against numpy's eigendecomposition: sizes around the LDS form's
+limits, numbers of operators on both sides of its limit, and matrices with zero
+reflectors, early deflation, exceptional shifts and extreme scales."""
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def eng(gpu_lib):
+    from muspinsim_amd.engine import SpinEngine
+    return SpinEngine("cuda:0")
+
+
+def _dev(a):
+    return torch.as_tensor(np.ascontiguousarray(a, dtype=complex)).cuda()
+
+
+def _matrices(rng, N):
+    G = rng.normal(size=(N, N)) + 1j * rng.normal(size=(N, N))
+    D = np.diag(np.arange(1, N + 1) * (0.1 + 0.2j))
+    block = G.copy()
+    block[N // 2:, : N // 2] = 0.0
+    cyc = np.roll(np.eye(N), 1, axis=0) + 0j       # every Wilkinson shift starts at zero
+    return [G, G + G.conj().T, -1j * (G + G.conj().T), D, D + np.triu(G, 1) / N, block, cyc,
+            1e100 * G, 1e-100 * G]
+
+
+@pytest.mark.parametrize("N", [4, 8, 9, 10, 16, 17, 36, 63, 64, 65])
+def test_amplitudes(eng, N):
+    rng = np.random.default_rng(N)
+    Ms = np.array(_matrices(rng, N))
+    for k in (1, 2, 3, 4):
+        r = rng.normal(size=(len(Ms), N)) + 1j * rng.normal(size=(len(Ms), N))
+        u = rng.normal(size=(len(Ms), k, N)) + 1j * rng.normal(size=(len(Ms), k, N))
+        lam, amp, c, _ = eng.lindblad_modes(_dev(Ms), _dev(r), _dev(u), want_c=True)
+        lam, amp = lam.cpu().numpy(), amp.cpu().numpy()
+        for b, M in enumerate(Ms):
+            w, V = np.linalg.eig(M)
+            cond = np.linalg.cond(V)
+            if cond > 1e6:
+                continue
+            s = np.abs(M).max()
+            # backward error of order N eps ||M||: eigenvalues to cond(V) times it
+            tol = 1e-15 * N * N * cond
+            assert np.abs(np.sort_complex(np.round(lam[b] / s, 9)) -
+                          np.sort_complex(np.round(w / s, 9))).max() <= max(tol, 3e-9)
+            # u^T f(M) r is independent of order and scaling of the modes
+            ref = np.linalg.solve(V, r[b])
+            for f in (lambda x: np.exp(x / s / N), lambda x: 1.0 / (x / s - 3.0j * N)):
+                want = (u[b] @ V) @ (ref * f(w))
+                got = amp[b] @ f(lam[b])
+                scale = np.abs(u[b]).sum(1) * np.abs(r[b]).max() * np.abs(f(w)).max()
+                assert np.all(np.abs(got - want) <= tol * scale)
+
+
+def test_zero_matrix_and_no_operators(eng):
+    N = 16
+    r = np.ones((1, N))
+    lam, _, c, _ = eng.lindblad_modes(_dev(np.zeros((1, N, N))), _dev(r), None, want_c=True)
+    assert np.all(lam.cpu().numpy() == 0) and np.allclose(c.cpu().numpy(), r)
