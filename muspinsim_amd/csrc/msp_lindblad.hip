@@ -173,35 +173,7 @@ __global__ void __launch_bounds__(NT) k_lindblad_modes(int N, double *Lg, const 
 // against 0.17 / 0.43, which keeps the one launch.  1024 Liouvillians of a
 // relaxing electron (N = 64): 8.4 against 3.2.
 
-__device__ inline double lane_f64(double v, int l)
-{
-    const long long x = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)(x & 0xffffffffll), l);
-    const int hi = __builtin_amdgcn_readlane((int)(x >> 32), l);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-__device__ inline cdbl lane_c(cdbl v, int l) { return cmk(lane_f64(v.re, l), lane_f64(v.im, l)); }
-
-// x <- [x lanes 0-31, y lanes 0-31], y <- [x lanes 32-63, y lanes 32-63]
-__device__ inline void swap32(double &x, double &y)
-{
-    const unsigned long long a = (unsigned long long)__double_as_longlong(x);
-    const unsigned long long b = (unsigned long long)__double_as_longlong(y);
-    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)a, (unsigned)b, false, false);
-    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(a >> 32), (unsigned)(b >> 32), false, false);
-    x = __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0]));
-    y = __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
-}
-// x <- [x row 0, y row 0, x row 2, y row 2], y <- [x row 1, y row 1, x row 3, y row 3]
-__device__ inline void swap16(double &x, double &y)
-{
-    const unsigned long long a = (unsigned long long)__double_as_longlong(x);
-    const unsigned long long b = (unsigned long long)__double_as_longlong(y);
-    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)a, (unsigned)b, false, false);
-    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(a >> 32), (unsigned)(b >> 32), false, false);
-    x = __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0]));
-    y = __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
-}
+__device__ inline cdbl lane_c(cdbl v, int l) { return cmk(readlane_f64(v.re, l), readlane_f64(v.im, l)); }
 
 // Sums over the 64 lanes of 16 doubles per lane, halving the values held per
 // step (by swaps of lane halves and rows, then by selects at the row mirror
@@ -580,7 +552,7 @@ __global__ void __launch_bounds__(64) k_lindblad_schur(int N, double *Lg, int n_
         for (int k = l; k < ihi; ++k) {
             const cdbl qn = S[bl + (k + 2 <= ihi ? k + 2 : k + 1)];
             if (lane > k + 1) qc = cmk(0.0, 0.0);
-            const double c = lane_f64(cv, k);
+            const double c = readlane_f64(cv, k);
             const cdbl s = lane_c(sv, k);
             // [p q] <- [c p + conj(s) q, -s p + c q]
             const cdbl t = rot_first(c, cconj(s), pc, qc);

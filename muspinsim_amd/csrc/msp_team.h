@@ -85,6 +85,37 @@ __device__ inline double dpp_f64(double v)
     return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
+// Lane l's double, in every lane (l wave-uniform).
+__device__ inline double readlane_f64(double v, int l)
+{
+    const long long x = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)(x & 0xffffffffll), l);
+    const int hi = __builtin_amdgcn_readlane((int)(x >> 32), l);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// Cross-lane swaps of gfx950 on the two halves of a double:
+//   swap32: x <- [x lanes 0-31, y lanes 0-31], y <- [x lanes 32-63, y lanes 32-63]
+//   swap16: x <- [x row 0, y row 0, x row 2, y row 2], y <- [x row 1, y row 1, x row 3, y row 3]
+__device__ inline void swap32(double &x, double &y)
+{
+    const unsigned long long a = (unsigned long long)__double_as_longlong(x);
+    const unsigned long long b = (unsigned long long)__double_as_longlong(y);
+    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)a, (unsigned)b, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(a >> 32), (unsigned)(b >> 32), false, false);
+    x = __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0]));
+    y = __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
+}
+__device__ inline void swap16(double &x, double &y)
+{
+    const unsigned long long a = (unsigned long long)__double_as_longlong(x);
+    const unsigned long long b = (unsigned long long)__double_as_longlong(y);
+    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)a, (unsigned)b, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(a >> 32), (unsigned)(b >> 32), false, false);
+    x = __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0]));
+    y = __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
+}
+
 // Sum over the 64 lanes of a wave on the VALU (no LDS traffic); the total is
 // exact in lane 63 only: pairs, quads, half rows, rows, then rows 0+1 and
 // 2+3 through row_bcast15 and the four rows through row_bcast31.

@@ -51,25 +51,6 @@ __device__ inline void lds_barrier()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-__device__ inline void swap32(double &x, double &y)
-{
-    const unsigned long long a = (unsigned long long)__double_as_longlong(x);
-    const unsigned long long b = (unsigned long long)__double_as_longlong(y);
-    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)a, (unsigned)b, false, false);
-    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(a >> 32), (unsigned)(b >> 32), false, false);
-    x = __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0]));
-    y = __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
-}
-__device__ inline void swap16(double &x, double &y)
-{
-    const unsigned long long a = (unsigned long long)__double_as_longlong(x);
-    const unsigned long long b = (unsigned long long)__double_as_longlong(y);
-    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)a, (unsigned)b, false, false);
-    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(a >> 32), (unsigned)(b >> 32), false, false);
-    x = __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0]));
-    y = __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
-}
-
 // Square root and its reciprocal of t > 0: hardware estimate, two coupled
 // Newton steps, and a last correction of the root.
 __device__ inline void sqrt_recip(double t, double &root, double &rec)
@@ -84,14 +65,6 @@ __device__ inline void sqrt_recip(double t, double &root, double &rec)
     }
     root = fma(fma(-gg, gg, t), h, gg);
     rec = 2.0 * h;
-}
-
-__device__ inline double readlane_f64(double v, int l)
-{
-    const long long x = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)(x & 0xffffffffll), l);
-    const int hi = __builtin_amdgcn_readlane((int)(x >> 32), l);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
 // Value of lane L of this lane's row of 16 lanes.
@@ -147,18 +120,18 @@ __global__ void __launch_bounds__(64 * W, OCC) k_tridiag_rt(int n, double *H, do
     cdbl *scal = R + 64 * W * NS;              // scale, tau scale, (-|tau scale|^2 / 2, -)
     double *dot = (double *)(scal + 3);
 
-    const int b0 = blockIdx.x;
     const int tid = threadIdx.x;
     const int lane = tid & 63, c = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    cdbl *A = (cdbl *)H + (size_t)b0 * n * n;
-    double *base = work + (size_t)b0 * dc_work_doubles(n);
+    cdbl *A = (cdbl *)H + (size_t)blockIdx.x * n * n;
+    double *base = work + (size_t)blockIdx.x * dc_work_doubles(n);
     double *e;
     cdbl *tau;
     dc_carve(n, base, &e, &tau);
-    double *d = E + (size_t)b0 * n;
+    double *d = E + (size_t)blockIdx.x * n;
 
     cdbl M[T::NSLOT];
+    double big = 0.0;
 #pragma unroll
     for (int a = 0; a < NS; ++a)
 #pragma unroll
@@ -171,10 +144,25 @@ __global__ void __launch_bounds__(64 * W, OCC) k_tridiag_rt(int n, double *H, do
                 if (row == cc) x.im = 0.0;
             }
             M[T::slot(a, J)] = x;
+            big = fmax(big, fmax(fabs(x.re), fabs(x.im)));
         }
+    // scaled by a power of two to a largest component near 1: x'^H A22 x' is
+    // cubic in the entries
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) big = fmax(big, __shfl_xor(big, o, 64));
+    if (lane == 0) dot[wave] = big;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < W; ++w) big = fmax(big, dot[w]);
+    int ex = 0;
+    if (big > 0.0 && big < INFINITY) (void)frexp(big, &ex);
+    ex = __builtin_amdgcn_readfirstlane(ex);
+#pragma unroll
+    for (int s = 0; s < T::NSLOT; ++s) M[s] = cmk(ldexp(M[s].re, -ex), ldexp(M[s].im, -ex));
     for (int i = tid; i < NP; i += 64 * W) {
         V[i] = Wv[i] = cmk(0.0, 0.0);
-        cn[i] = (i < n) ? A[(size_t)i * n] : cmk(0.0, 0.0);
+        const cdbl x = (i < n) ? A[(size_t)i * n] : cmk(0.0, 0.0);
+        cn[i] = cmk(ldexp(x.re, -ex), ldexp(x.im, -ex));
     }
     for (int i = tid; i < W * NP + 64 * W * NS; i += 64 * W) P[i] = cmk(0.0, 0.0);
     // LDS places of this lane: its rows and columns, its share of the sums
@@ -222,7 +210,7 @@ __global__ void __launch_bounds__(64 * W, OCC) k_tridiag_rt(int n, double *H, do
                 const cdbl a = cmk(readlane_f64(x[t].re, (k + 1) & 63), readlane_f64(x[t].im, (k + 1) & 63));
                 if (((k + 1) >> 6) == t) alpha = a;
             }
-            if (lane == (k & 63)) d[k] = dk;
+            if (lane == (k & 63)) d[k] = ldexp(dk, ex);
             if (k == n - 1) break;
             const double xn2 = wave_sum_all(part);
             cdbl tk = cmk(0.0, 0.0), scale = tk, xh = tk;
@@ -250,7 +238,7 @@ __global__ void __launch_bounds__(64 * W, OCC) k_tridiag_rt(int n, double *H, do
                 scal[0] = scale;
                 scal[1] = u;
                 scal[2] = cmk(-0.5 * cabs2(u), 0.0);
-                e[k] = beta;
+                e[k] = ldexp(beta, ex);
                 tau[k] = tk;
             }
             __builtin_amdgcn_s_setprio(0);
