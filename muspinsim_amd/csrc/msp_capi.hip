@@ -195,6 +195,9 @@ int msp_eigh(int n, int batch, double *d_H, double *d_E, double *d_U, int32_t *d
     if (batch < 0) return fail(MSP_ERR_VALUE, "msp_eigh: batch < 0");
     if (batch == 0) return MSP_OK;
     if (!d_H || !d_E || !d_U || !d_info) return fail(MSP_ERR_VALUE, "msp_eigh: null pointer");
+    // (neither choice for n <= kJacobiMax needs a workspace)
+    if (method == MSP_EIGH_AUTO && n <= kSmallMax)
+        return hip_status(launch_eigh_small(n, batch, d_H, d_E, d_U, d_info, S(stream)), "msp_eigh(small)");
     if (method == MSP_EIGH_AUTO) method = (n <= kJacobiMax) ? MSP_EIGH_JACOBI : MSP_EIGH_DC;
     if (method == MSP_EIGH_JACOBI) {
         if (n > kJacobiMax)
@@ -262,6 +265,9 @@ int msp_eigh_noalloc(int n, int batch, double *d_H, double *d_E, double *d_U, in
     if (batch < 0) return fail(MSP_ERR_VALUE, "msp_eigh_noalloc: batch < 0");
     if (batch == 0) return MSP_OK;
     if (!d_H || !d_E || !d_U || !d_info) return fail(MSP_ERR_VALUE, "msp_eigh_noalloc: null pointer");
+    // (neither choice for n <= kJacobiMax needs a workspace)
+    if (method == MSP_EIGH_AUTO && n <= kSmallMax)
+        return hip_status(launch_eigh_small(n, batch, d_H, d_E, d_U, d_info, S(stream)), "msp_eigh_noalloc(small)");
     if (method == MSP_EIGH_AUTO) method = (n <= kJacobiMax) ? MSP_EIGH_JACOBI : MSP_EIGH_DC;
     if (method == MSP_EIGH_JACOBI) {
         if (n > kJacobiMax)

@@ -36,6 +36,12 @@ hipError_t launch_build_h(int n, int batch, const MspSystem *systems, const MspT
                           int lower, double *H, hipStream_t s);
 hipError_t launch_eigh_jacobi(int n, int batch, const double *H, double *E, double *U,
                               int32_t *info, int max_sweeps, hipStream_t s);
+// One-launch Jacobi eigensolver for n <= kSmallMax (a wave or less per matrix, lower triangle
+// read, H left as it is, no workspace).
+constexpr int kSmallMax = 16;
+hipError_t launch_eigh_small(int n, int batch, const double *H, double *E, double *U, int32_t *info,
+                             hipStream_t s);
+// n <= kSmallMax takes launch_eigh_small.
 // overlap: form the WY factors on a per-thread side stream while the divide
 // and conquer runs (forked from and joined back into s); false keeps every
 // launch on s and creates no events.

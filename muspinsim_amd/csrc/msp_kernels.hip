@@ -1124,6 +1124,7 @@ static hipError_t eigh_dc_middle(int n, int batch, double *H, double *E, int32_t
 hipError_t launch_eigh_dc(int n, int batch, double *H, double *E, double *U, int32_t *info,
                           double *work, hipStream_t s, bool overlap)
 {
+    if (n <= kSmallMax) return launch_eigh_small(n, batch, H, E, U, info, s);
     hipError_t err = hipSuccess;
     if (n <= 1024) {
         ProfScope ps_("k_tridiag", s);

@@ -188,6 +188,10 @@ class SpinEngine:
         m = autotune.eigh_method(self.tuning, n, count)
         if m == N.MSP_EIGH_JACOBI and n > 64:
             m = N.MSP_EIGH_AUTO
+        if m == N.MSP_EIGH_AUTO and 16 < n <= 64:
+            # msp_eigh's own choice here is the LDS Jacobi kernel, which needs
+            # no workspace; with one, divide and conquer is faster
+            m = N.MSP_EIGH_DC
         return m
 
     def per_instance_bytes(self, n, complex_rho, method=None):

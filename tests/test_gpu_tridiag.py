@@ -1,6 +1,7 @@
-"""Register-resident Householder tridiagonalisation (through msp_eigh's divide
-and conquer) at the edges of its strips and column blocks, on structured
-matrices and on both sides of its batch rule."""
+"""Hermitian eigensolver at the edges of its kernels: the one-wave Jacobi kernel
+(n <= 16) and, through the divide and conquer, the register-resident Householder
+tridiagonalisation (n <= 192), on structured matrices and on both sides of its
+batch rule."""
 
 import numpy as np
 import pytest
@@ -20,14 +21,15 @@ def _herm(rng, n):
     return (X + X.conj().T) / 2
 
 
-def _check(eng, Hs):
+def _check(eng, Hs, method=None):
     """Backward error of order n eps ||H|| and orthonormal eigenvectors; the
     strict upper triangle, which the solver must not read, is NaN."""
     from muspinsim_amd import _native as N
     n = Hs.shape[1]
     low = Hs.copy()
     low[:, np.triu_indices(n, 1)[0], np.triu_indices(n, 1)[1]] = np.nan
-    E, U, info = eng.eigh(torch.as_tensor(low).cuda(), method=N.MSP_EIGH_DC)
+    E, U, info = eng.eigh(torch.as_tensor(low).cuda(),
+                          method=N.MSP_EIGH_DC if method is None else method)
     E, U = E.cpu().numpy(), U.cpu().numpy()
     assert np.all(info.cpu().numpy() == 0)
     nrm = np.maximum(np.abs(E).max(1), 1e-300)
@@ -37,7 +39,7 @@ def _check(eng, Hs):
     assert np.abs(UU - np.eye(n)).max() <= 1e-14 * max(n, 10)
 
 
-@pytest.mark.parametrize("n", [1, 2, 3, 11, 12, 13, 15, 16, 17, 24, 25, 31, 32, 33, 48, 49, 64, 65,
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 7, 8, 9, 11, 12, 13, 15, 16, 17, 24, 25, 31, 32, 33, 48, 49, 64, 65,
                                80, 81, 95, 96, 97, 108, 112, 113, 127, 128, 129, 160, 161, 191,
                                192, 193])
 def test_structured(eng, n):
@@ -50,9 +52,15 @@ def test_structured(eng, n):
     half = np.zeros((n, n), dtype=complex)     # two uncoupled blocks: a zero column on the way
     m = n // 2
     half[:m, :m], half[m:, m:] = _herm(rng, m), _herm(rng, n - m)
-    _check(eng, np.array([_herm(rng, n), 1e6 * _herm(rng, n), np.zeros((n, n)) + 0j,
-                          np.diag(rng.normal(size=n)) + 0j, tri, np.outer(v, v.conj()),
-                          _herm(rng, n).real + 0j, half]))
+    Hs = np.array([_herm(rng, n), 1e6 * _herm(rng, n), np.zeros((n, n)) + 0j,
+                   np.diag(rng.normal(size=n)) + 0j, tri, np.outer(v, v.conj()),
+                   _herm(rng, n).real + 0j, half,
+                   1e-120 * _herm(rng, n), 1e120 * _herm(rng, n)])
+    _check(eng, Hs)
+    if n <= 16:
+        from muspinsim_amd import _native as N
+        _check(eng, Hs, N.MSP_EIGH_AUTO)
+        _check(eng, Hs[:1], N.MSP_EIGH_AUTO)
 
 
 @pytest.mark.parametrize("n", [40, 90])
