@@ -97,7 +97,7 @@ class PolarisationModel:
                     N.check(L.msp_build_h(n, nb, plan.d_sys.data_ptr(), plan.d_terms.data_ptr(),
                                           p(g.sid), g.Br.data_ptr(), None, 1, g.H.data_ptr(), st))
                 N.check(L.msp_eigh(n, nb, g.H.data_ptr(), g.E.data_ptr(), g.U.data_ptr(),
-                                   g.info.data_ptr(), eng.method, g.work.data_ptr(), g.wsb, st))
+                                   g.info.data_ptr(), g.method, g.work.data_ptr(), g.wsb, st))
                 Y = g.H
                 N.check(L.msp_apply_muon_op(n, nb, plan.d_sys.data_ptr(), p(g.sid),
                                             g.pr.data_ptr(), 1, g.U.data_ptr(), Y.data_ptr(), st))
