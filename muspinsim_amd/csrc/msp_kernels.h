@@ -94,7 +94,7 @@ std::string prof_report();
 // Householder tridiagonalisation for n <= 1024, kernel chosen by n.
 hipError_t launch_tridiag(int n, int batch, double *H, double *E, double *work, hipStream_t s);
 // Register-resident reduction (matrix in VGPRs, one workgroup per matrix) for
-// n <= 192, same outputs as the panel kernel.
+// n <= 256, same outputs as the panel kernel.
 hipError_t launch_tridiag_rt(int n, int batch, double *H, double *E, double *work, hipStream_t s);
 // U = Q Z on MFMA.  off: rows between a reflector's column and its unit
 // element (1 for the one-stage reduction, 16 for the band stage's panels);

@@ -453,8 +453,7 @@ hipError_t lp_launch(int n, int batch, double *H, double *E, double *work, hipSt
 // lower-triangle panel kernel above (panels in the workspace from n = 513 on).
 hipError_t launch_tridiag(int n, int batch, double *H, double *E, double *work, hipStream_t s)
 {
-    if (n <= 192) return launch_tridiag_rt(n, batch, H, E, work, s);
-    if (n <= 256) return lp_launch<MSP_TD_WL, 8, 4, 4>(n, batch, H, E, work, s);
+    if (n <= 256) return launch_tridiag_rt(n, batch, H, E, work, s);
     if (n <= 512) return lp_launch<MSP_TD_WL, 4, 8, 4>(n, batch, H, E, work, s);
     if (n <= 1024) return lp_launch<MSP_TD_WL, MSP_TD_NBL, 16, MSP_TD_RB1024, true>(n, batch, H, E, work, s);
     return hipErrorNotSupported;

@@ -1,5 +1,5 @@
 // Householder tridiagonalisation with the matrix resident in the registers of
-// one CU (gfx950, n <= 192).  Same reduction and outputs as the panel kernel
+// one CU (gfx950, n <= 256).  Same reduction and outputs as the panel kernel
 // (msp_tridiag_lp.hip): reflectors v with v_{k+1} = 1, tails below the
 // subdiagonal of the row-major matrix, d to E, e and tau to the workspace.
 //
@@ -8,6 +8,9 @@
 // the strip's diagonal region, which is held whole.  Every wave has the same
 // static code and the same share of the live matrix at every step; row sums
 // stay in one wave, column sums cross the W waves once per step through LDS.
+// Above n = 192 the registers hold the trailing 192 columns; the one or two
+// pairs of 16-column blocks before them stay in global memory, updated there
+// (each element by one lane) until their 32 or 64 columns are done.
 //
 // Column step k:
 //   1. wave 0 brings column k up to date and forms its reflector, the others
@@ -29,7 +32,8 @@
 // kernel (below n = 65: registers in 64-column slots) against this one:
 //   n = 192 18.6 / 10.3, 144 10.7 / 6.6, 128 8.3 / 3.2, 108 6.2 / 2.5,
 //   96 5.1 / 1.7, 72 3.3 / 1.1, 64 2.25 / 0.74, 48 1.82 / 0.37, 32 0.91 / 0.19,
-//   16 0.47 / 0.06; one matrix: n = 192 1.88 / 0.62, 64 0.18 / 0.11.
+//   16 0.47 / 0.06; one matrix: n = 192 1.88 / 0.62, 64 0.18 / 0.11; n = 256
+//   3.3 / 1.65, and for 256 matrices 3.7 / 2.3.
 // Measured and not taken: 16 x 16 tiles in MFMA accumulators dealt to the waves
 // with the rank-2 update on MFMA (n = 192 14.6 ms: FP64 MFMA and FP64 VALU
 // share one pipe, so the products delay the other waves' serial chains, and a
@@ -74,6 +78,18 @@ __device__ inline double row_bcast(double v)
     return __longlong_as_double(
         __builtin_amdgcn_update_dpp(0ll, __double_as_longlong(v), 0x150 + L, 0xF, 0xF, true));
 }
+// m -= v w^H + w v^H at one element, as FMA chains
+__device__ __forceinline__ void rank2(cdbl &m, cdbl vi, cdbl wi, cdbl vj, cdbl wj)
+{
+    m.re = fma(-vi.re, wj.re, m.re);
+    m.im = fma(-vi.im, wj.re, m.im);
+    m.re = fma(-vi.im, wj.im, m.re);
+    m.im = fma(vi.re, wj.im, m.im);
+    m.re = fma(-wi.re, vj.re, m.re);
+    m.im = fma(-wi.im, vj.re, m.im);
+    m.re = fma(-wi.im, vj.im, m.re);
+    m.im = fma(wi.re, vj.im, m.im);
+}
 // o[a] = x of lane FIRST + STEP a of each row of 16 lanes
 template <int FIRST, int STEP, int NS, int... I>
 __device__ inline void spread(cdbl x, cdbl (&o)[NS], std::integer_sequence<int, I...>)
@@ -82,7 +98,10 @@ __device__ inline void spread(cdbl x, cdbl (&o)[NS], std::integer_sequence<int, 
 }
 
 // W: waves, NS: strips of 4 W rows (n <= 4 W NS), OCC: waves per SIMD asked for.
-template <int W, int NS>
+// JC: pairs of leading 16-column blocks that are kept in place in global memory
+// (the matrix's own, read and written by the lanes that would hold them) while
+// their columns last.
+template <int W, int NS, int JC>
 struct RtShape {
     static constexpr int SR = 4 * W;                       // rows per strip
     static constexpr int NR = SR * NS;
@@ -92,11 +111,11 @@ struct RtShape {
     static constexpr int slot(int a, int J)
     {
         int s = 0;
-        for (int b = 0; b < a; ++b) s += dl(b) + 1;
-        return s + J;
+        for (int b = 0; b < a; ++b) s += dl(b) + 1 > 2 * JC ? dl(b) + 1 - 2 * JC : 0;
+        return s + J - 2 * JC;
     }
     static constexpr int NJ = dl(NS - 1) + 1;
-    static constexpr int NSLOT = slot(NS, 0);
+    static constexpr int NSLOT = slot(NS, 2 * JC);
     static constexpr int NC = (NR + 63) / 64;              // entries per lane of a vector
     static constexpr int NP = 64 * NC;
     // LDS: x', column k + 1, v and w, column sums per wave, row sums per lane,
@@ -105,12 +124,13 @@ struct RtShape {
     static constexpr size_t LDS = sizeof(cdbl) * CDBL + sizeof(double) * ((W + 1) & ~1);
 };
 
-template <int W, int NS, int OCC>
+template <int W, int NS, int OCC, int JC>
 __global__ void __launch_bounds__(64 * W, OCC) k_tridiag_rt(int n, double *H, double *E, double *work)
 {
-    using T = RtShape<W, NS>;
+    using T = RtShape<W, NS, JC>;
     constexpr int SR = T::SR, NJ = T::NJ, NC = T::NC, NP = T::NP;
     static_assert(NS <= 8, "two lanes per row of a wave");
+    static_assert(JC == 0 || W == 8, "a strip's diagonal region is one pair of blocks");
     extern __shared__ __align__(16) unsigned char smem[];
     cdbl *col = (cdbl *)smem;                  // x': zero up to row k
     cdbl *cn = col + NP;                       // column k + 1 before step k's update
@@ -132,20 +152,23 @@ __global__ void __launch_bounds__(64 * W, OCC) k_tridiag_rt(int n, double *H, do
 
     cdbl M[T::NSLOT];
     double big = 0.0;
+    const auto element = [&](int row, int cc) {
+        cdbl x = cmk(0.0, 0.0);
+        if (row < n && cc < n) {
+            x = (row >= cc) ? A[(size_t)row * n + cc] : A[(size_t)cc * n + row];
+            if (row < cc) x.im = -x.im;
+            if (row == cc) x.im = 0.0;
+        }
+        big = fmax(big, fmax(fabs(x.re), fabs(x.im)));
+        return x;
+    };
 #pragma unroll
     for (int a = 0; a < NS; ++a)
 #pragma unroll
-        for (int J = 0; J <= T::dl(a); ++J) {
-            const int row = SR * a + 4 * wave + g, cc = 16 * J + c;
-            cdbl x = cmk(0.0, 0.0);
-            if (row < n && cc < n) {
-                x = (row >= cc) ? A[(size_t)row * n + cc] : A[(size_t)cc * n + row];
-                if (row < cc) x.im = -x.im;
-                if (row == cc) x.im = 0.0;
-            }
-            M[T::slot(a, J)] = x;
-            big = fmax(big, fmax(fabs(x.re), fabs(x.im)));
-        }
+        for (int J = 2 * JC; J <= T::dl(a); ++J)
+            M[T::slot(a, J)] = element(SR * a + 4 * wave + g, 16 * J + c);
+    for (int a = 0; a < NS; ++a)
+        for (int J = 0; J < 2 * JC && J <= T::dl(a); ++J) (void)element(SR * a + 4 * wave + g, 16 * J + c);
     // scaled by a power of two to a largest component near 1: x'^H A22 x' is
     // cubic in the entries
 #pragma unroll
@@ -163,6 +186,31 @@ __global__ void __launch_bounds__(64 * W, OCC) k_tridiag_rt(int n, double *H, do
         V[i] = Wv[i] = cmk(0.0, 0.0);
         const cdbl x = (i < n) ? A[(size_t)i * n] : cmk(0.0, 0.0);
         cn[i] = cmk(ldexp(x.re, -ex), ldexp(x.im, -ex));
+    }
+    if constexpr (JC > 0) {
+        // scaled in place; the diagonal regions made whole (the mirror of an
+        // element below the diagonal is another lane's, so all are read before
+        // any is written)
+        cdbl cold[2 * JC * JC];
+#pragma unroll
+        for (int a = 0; a < JC; ++a)
+#pragma unroll
+            for (int J = 0; J < 2 * JC && J <= T::dl(a); ++J)
+                cold[2 * JC * a + J] = element(SR * a + 4 * wave + g, 16 * J + c);
+        __syncthreads();
+        const auto put = [&](int row, int J, cdbl x) {
+            if (row < n) A[(size_t)row * n + 16 * J + c] = cmk(ldexp(x.re, -ex), ldexp(x.im, -ex));
+        };
+#pragma unroll
+        for (int a = 0; a < JC; ++a)
+#pragma unroll
+            for (int J = 0; J < 2 * JC && J <= T::dl(a); ++J)
+                put(SR * a + 4 * wave + g, J, cold[2 * JC * a + J]);
+        for (int a = JC; a < NS; ++a)
+            for (int J = 0; J < 2 * JC; ++J) {
+                const int row = SR * a + 4 * wave + g;
+                put(row, J, row < n ? A[(size_t)row * n + 16 * J + c] : cmk(0.0, 0.0));
+            }
     }
     for (int i = tid; i < W * NP + 64 * W * NS; i += 64 * W) P[i] = cmk(0.0, 0.0);
     // LDS places of this lane: its rows and columns, its share of the sums
@@ -250,29 +298,52 @@ __global__ void __launch_bounds__(64 * W, OCC) k_tridiag_rt(int n, double *H, do
         // pending update A22 -= v w^H + w v^H of the live blocks
         if (k > 0) {
             // lane c of a row of 16 reads v (c even) or w (c odd) of strip c / 2
-            cdbl vr[NS], wr[NS];
             const cdbl ro = *vrp;
+            if constexpr (JC > 0) {
+                // blocks in global memory, a pair per strip, the next strip's
+                // loads issued before this strip's stores; finished columns hold
+                // reflector tails, which the lanes leave alone
+#pragma unroll 1
+                for (int jp = jp1; jp < JC; ++jp) {
+                    const cdbl v0 = V[32 * jp + c], w0 = Wv[32 * jp + c];
+                    const cdbl v1 = V[32 * jp + 16 + c], w1 = Wv[32 * jp + 16 + c];
+                    const bool l0 = 32 * jp + c > k, l1 = 32 * jp + 16 + c > k;
+                    int row = SR * jp + 4 * wave + g;
+                    cdbl *p0 = A + row * n + 32 * jp + c;
+                    cdbl y0 = cmk(0.0, 0.0), y1 = y0;
+                    if (row < n) {
+                        y0 = p0[0];
+                        y1 = p0[16];
+                    }
+#pragma unroll 1
+                    for (int a = jp; a < NS; ++a) {
+                        cdbl x0 = y0, x1 = y1, *pn = p0 + SR * n;
+                        if (row + SR < n) {
+                            y0 = pn[0];
+                            y1 = pn[16];
+                        }
+                        const cdbl va = V[row], wa = Wv[row];
+                        rank2(x0, va, wa, v0, w0);
+                        rank2(x1, va, wa, v1, w1);
+                        if (row < n && l0) p0[0] = x0;
+                        if (row < n && l1) p0[16] = x1;
+                        row += SR;
+                        p0 = pn;
+                    }
+                }
+            }
+            cdbl vr[NS], wr[NS];
             spread<0, 2>(ro, vr, std::make_integer_sequence<int, NS>());
             spread<1, 2>(ro, wr, std::make_integer_sequence<int, NS>());
 #pragma unroll
-            for (int jp = 0; jp < (NJ + 1) / 2; ++jp) {
+            for (int jp = JC; jp < (NJ + 1) / 2; ++jp) {
                 if (jp < jp1) continue;
 #pragma unroll
                 for (int J = 2 * jp; J < 2 * jp + 2 && J < NJ; ++J) {
                     const cdbl vj = V[16 * J + c], wj = Wv[16 * J + c];
 #pragma unroll
-                    for (int a = 0; a < NS; ++a) {
-                        if (J > T::dl(a)) continue;
-                        cdbl &m = M[T::slot(a, J)];
-                        m.re = fma(-vr[a].re, wj.re, m.re);
-                        m.im = fma(-vr[a].im, wj.re, m.im);
-                        m.re = fma(-vr[a].im, wj.im, m.re);
-                        m.im = fma(vr[a].re, wj.im, m.im);
-                        m.re = fma(-wr[a].re, vj.re, m.re);
-                        m.im = fma(-wr[a].im, vj.re, m.im);
-                        m.re = fma(-wr[a].im, vj.im, m.re);
-                        m.im = fma(wr[a].re, vj.im, m.im);
-                    }
+                    for (int a = 0; a < NS; ++a)
+                        if (J <= T::dl(a)) rank2(M[T::slot(a, J)], vr[a], wr[a], vj, wj);
                 }
             }
         }
@@ -284,9 +355,58 @@ __global__ void __launch_bounds__(64 * W, OCC) k_tridiag_rt(int n, double *H, do
             double dacc = 0.0;
 #pragma unroll
             for (int a = 0; a < NS; ++a) rs[a] = cmk(0.0, 0.0);
-            spread<0, 1>(*xrp, xr, std::make_integer_sequence<int, NS>());
+            const cdbl xo = *xrp;
+            const auto column_sums = [&](int jp, cdbl (&cs)[2]) {
+                swap32(cs[0].re, cs[1].re);
+                swap32(cs[0].im, cs[1].im);
+                double s = cs[0].re + cs[1].re, t = cs[0].im + cs[1].im;
+                swap16(s, t);
+                Pw[64 * jp] = s + t;
+            };
+            if constexpr (JC > 0) {
+#pragma unroll 1
+                for (int jp = jp1; jp < JC; ++jp) {
+                    const cdbl xc0 = col[32 * jp + c], xc1 = col[32 * jp + 16 + c];
+                    const bool next0 = k + 1 == 32 * jp + c, next1 = k + 1 == 32 * jp + 16 + c;
+                    int row = SR * jp + 4 * wave + g;
+                    const cdbl *p0 = A + row * n + 32 * jp + c;
+                    cdbl y0 = cmk(0.0, 0.0), y1 = y0, cs[2];
+                    cs[0] = cs[1] = y0;
+                    if (row < n) {
+                        y0 = p0[0];
+                        y1 = p0[16];
+                    }
+#pragma unroll 1
+                    for (int a = jp; a < NS; ++a) {
+                        const cdbl x0 = row < n ? y0 : cmk(0.0, 0.0), x1 = row < n ? y1 : cmk(0.0, 0.0);
+                        p0 += SR * n;
+                        if (row + SR < n) {
+                            y0 = p0[0];
+                            y1 = p0[16];
+                        }
+                        const cdbl xa = col[row];
+                        if (next0) cn[row] = x0;
+                        if (next1) cn[row] = x1;
+                        cdbl r = cmk(0.0, 0.0);
+                        cfma(r, x0, xc0);
+                        cfma(r, x1, xc1);
+                        const double t = fma(xa.re, r.re, xa.im * r.im);
+                        dacc += t;
+                        if (a > jp) {          // (strip jp: its diagonal region)
+                            dacc += t;
+                            cfmac(cs[0], x0, xa);
+                            cfmac(cs[1], x1, xa);
+                        }
+                        // a strip's row sums collect in its place in R
+                        Rw[64 * a] = jp > jp1 ? cadd(Rw[64 * a], r) : r;
+                        row += SR;
+                    }
+                    column_sums(jp, cs);
+                }
+            }
+            spread<0, 1>(xo, xr, std::make_integer_sequence<int, NS>());
 #pragma unroll
-            for (int jp = 0; jp < (NJ + 1) / 2; ++jp) {
+            for (int jp = JC; jp < (NJ + 1) / 2; ++jp) {
                 if (jp < jp1) continue;
                 cdbl cs[2];
                 cs[0] = cs[1] = cmk(0.0, 0.0);
@@ -313,23 +433,23 @@ __global__ void __launch_bounds__(64 * W, OCC) k_tridiag_rt(int n, double *H, do
                             if (J <= T::dl(a)) cn[SR * a + 4 * wave + g] = M[T::slot(a, J)];
                     }
                 }
-                if (2 * jp < T::j0(NS - 1)) {
-                    swap32(cs[0].re, cs[1].re);
-                    swap32(cs[0].im, cs[1].im);
-                    double s = cs[0].re + cs[1].re, t = cs[0].im + cs[1].im;
-                    swap16(s, t);
-                    Pw[64 * jp] = s + t;
-                }
+                if (2 * jp < T::j0(NS - 1)) column_sums(jp, cs);
             }
 #pragma unroll
             for (int a = 0; a < NS; ++a) dacc = fma(xr[a].re, rs[a].re, fma(xr[a].im, rs[a].im, dacc));
             // row sums of the live strips, left to stage 3 (this wave's rows)
-            if (k + 1 < SR * (NS / 2)) {
+            if (JC > 0 && jp1 < JC) {
 #pragma unroll
-                for (int a = 0; a < NS / 2; ++a) Rw[64 * a] = rs[a];
+                for (int a = 0; a < NS; ++a)
+                    if (T::dl(a) >= 2 * JC) Rw[64 * a] = cadd(Rw[64 * a], rs[a]);
+            } else {
+                if (k + 1 < SR * (NS / 2)) {
+#pragma unroll
+                    for (int a = 0; a < NS / 2; ++a) Rw[64 * a] = rs[a];
+                }
+#pragma unroll
+                for (int a = NS / 2; a < NS; ++a) Rw[64 * a] = rs[a];
             }
-#pragma unroll
-            for (int a = NS / 2; a < NS; ++a) Rw[64 * a] = rs[a];
             dacc = wave_sum_all(dacc);
             if (lane == 0) dot[wave] = dacc;
         }
@@ -369,13 +489,13 @@ __global__ void __launch_bounds__(64 * W, OCC) k_tridiag_rt(int n, double *H, do
     }
 }
 
-template <int W, int NS, int OCC>
+template <int W, int NS, int OCC, int JC = 0>
 hipError_t rt_launch(int n, int batch, double *H, double *E, double *work, hipStream_t s)
 {
-    const size_t lds = RtShape<W, NS>::LDS;
-    hipError_t err = msp_set_lds((const void *)k_tridiag_rt<W, NS, OCC>, lds);
+    const size_t lds = RtShape<W, NS, JC>::LDS;
+    hipError_t err = msp_set_lds((const void *)k_tridiag_rt<W, NS, OCC, JC>, lds);
     if (err != hipSuccess) return err;
-    hipLaunchKernelGGL((k_tridiag_rt<W, NS, OCC>), dim3(batch), dim3(64 * W), lds, s, n, H, E, work);
+    hipLaunchKernelGGL((k_tridiag_rt<W, NS, OCC, JC>), dim3(batch), dim3(64 * W), lds, s, n, H, E, work);
     return hipGetLastError();
 }
 
@@ -391,6 +511,7 @@ hipError_t rt_launch(int n, int batch, double *H, double *E, double *work, hipSt
 // 0.37; n = 96 at two workgroups per CU 0.205 / 1.93, at three (four registers
 // spilled) 0.230 / 1.71; n = 32 two waves 0.051 / 0.19, one 0.058 / 0.19;
 // n = 128 four waves 0.32 / 3.1, eight 0.31 / 4.9.
+// Above n = 256 the columns left in global memory would be most of the work.
 hipError_t launch_tridiag_rt(int n, int batch, double *H, double *E, double *work, hipStream_t s)
 {
     const bool many = batch > 512;
@@ -408,5 +529,7 @@ hipError_t launch_tridiag_rt(int n, int batch, double *H, double *E, double *wor
     if (n <= 128) return rt_launch<4, 8, 2>(n, batch, H, E, work, s);
     if (n <= 160) return rt_launch<8, 5, 2>(n, batch, H, E, work, s);
     if (n <= 192) return rt_launch<8, 6, 2>(n, batch, H, E, work, s);
+    if (n <= 224) return rt_launch<8, 7, 2, 1>(n, batch, H, E, work, s);
+    if (n <= 256) return rt_launch<8, 8, 2, 2>(n, batch, H, E, work, s);
     return hipErrorNotSupported;
 }

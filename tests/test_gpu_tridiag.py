@@ -1,6 +1,6 @@
 """Hermitian eigensolver at the edges of its kernels: the one-wave Jacobi kernel
 (n <= 16) and, through the divide and conquer, the register-resident Householder
-tridiagonalisation (n <= 192), on structured matrices and on both sides of its
+tridiagonalisation (n <= 256), on structured matrices and on both sides of its
 batch rule."""
 
 import numpy as np
@@ -41,7 +41,7 @@ def _check(eng, Hs, method=None):
 
 @pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 7, 8, 9, 11, 12, 13, 15, 16, 17, 24, 25, 31, 32, 33, 48, 49, 64, 65,
                                80, 81, 95, 96, 97, 108, 112, 113, 127, 128, 129, 160, 161, 191,
-                               192, 193])
+                               192, 193, 200, 223, 224, 225, 255, 256, 257])
 def test_structured(eng, n):
     rng = np.random.default_rng(n)
     tri = np.diag(rng.normal(size=n)) + 0j
