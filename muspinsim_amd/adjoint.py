@@ -21,7 +21,7 @@ import torch
 
 from . import _native as N
 from . import gpu
-from .engine import SystemDesc
+from .engine import SystemDesc, pack_systems
 
 
 class PolarisationModel:
@@ -56,12 +56,18 @@ class PolarisationModel:
 
     def dH(self, theta, system):
         """(nparam, n, n) complex derivative Hamiltonians on the device."""
-        mats = []
-        for terms in self.dterms(np.asarray(theta, dtype=float)):
-            desc = SystemDesc(Is=list(system.Is), gammas=list(system.gammas), terms=list(terms),
-                              muon_index=system.muon_index)
-            mats.append(gpu.build_h(desc))
-        return gpu.to_dev(np.array(mats))
+        eng = self.engine
+        descs = [SystemDesc(Is=list(system.Is), gammas=list(system.gammas), terms=list(terms),
+                            muon_index=system.muon_index)
+                 for terms in self.dterms(np.asarray(theta, dtype=float))]
+        n = system.n
+        H = torch.empty((len(descs), n, n), dtype=torch.complex128, device=eng.device)
+        if descs:
+            dsys, dterms, ids = eng._upload(*pack_systems(descs),
+                                            np.arange(len(descs), dtype=np.int32))
+            N.check(eng.lib.msp_build_h(n, len(descs), dsys.data_ptr(), dterms.data_ptr(),
+                                        ids.data_ptr(), None, None, 0, H.data_ptr(), eng.stream()))
+        return H
 
     def vjp(self, theta, grad):
         """dL/dtheta (numpy, nparam) for upstream grad = dL/dresults (n_slots, T)."""

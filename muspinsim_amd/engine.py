@@ -175,6 +175,27 @@ class SpinEngine:
     def _dev(self, a, dtype=torch.float64):
         return torch.as_tensor(np.ascontiguousarray(a), dtype=dtype).to(self.device)
 
+    def _upload(self, *arrays):
+        """The arrays on the device, packed into one transfer (each a view of
+        one buffer, 256-byte aligned): a plan is a dozen small arrays, and a
+        transfer costs as much as the array up to about 100 KB."""
+        arrays = [np.ascontiguousarray(a) for a in arrays]
+        offs, total = [], 0
+        for a in arrays:
+            offs.append(total)
+            total += -(-a.nbytes // 256) * 256
+        buf = np.zeros(max(total, 1), dtype=np.uint8)
+        for a, o in zip(arrays, offs):
+            buf[o:o + a.nbytes] = np.frombuffer(a.tobytes(), dtype=np.uint8)
+        dev = torch.from_numpy(buf).to(self.device)
+        out = []
+        for a, o in zip(arrays, offs):
+            t = dev[o:o + a.nbytes]
+            if a.dtype.names is None:
+                t = t.view(getattr(torch, str(a.dtype))).reshape(a.shape)
+            out.append(t)
+        return out
+
     def _bytes_view(self, structarr):
         raw = np.frombuffer(np.ascontiguousarray(structarr).tobytes(), dtype=np.uint8)
         return torch.from_numpy(raw.copy()).to(self.device)
@@ -332,15 +353,20 @@ class SpinEngine:
         with np.errstate(divide="ignore", invalid="ignore"):
             check = (cnst.e * (cnst.hbar ** 2) * Bn) / (2 * cnst.m_p * cnst.k * Tarr)
         iso = check == 0                       # every non-muon spin at infinite temperature
-        mu_first = np.array([systems[int(k)].muon_index == 0 for k in batch.sys_id])
-        lind = np.array([bool(systems[int(k)].dissip) for k in batch.sys_id])
+        sid = np.asarray(batch.sys_id, dtype=np.int64)
+        mu_first = np.array([s.muon_index == 0 for s in systems])[sid]
+        lind = np.array([bool(s.dissip) for s in systems])[sid]
         fast = iso & mu_first & (batch.y == "asymmetry") & ~lind
         iso = iso & ~lind
-        ns = np.array([systems[int(k)].n for k in batch.sys_id])
+        ns = np.array([s.n for s in systems])[sid]
         sysarr, termarr = pack_systems(systems)
-        plan.d_sys = self._bytes_view(sysarr)
-        plan.d_terms = self._bytes_view(termarr)
-        plan.times = self._dev(batch.times if batch.y == "asymmetry" else np.zeros(1))
+        order = np.argsort(batch.slot, kind="stable")
+        counts = np.bincount(batch.slot, minlength=batch.n_slots)
+        ptr = np.concatenate([[0], np.cumsum(counts)])
+        plan.d_sys, plan.d_terms, plan.times, plan.d_ptr, plan.d_order = self._upload(
+            sysarr, termarr,
+            np.asarray(batch.times if batch.y == "asymmetry" else np.zeros(1), dtype=float),
+            ptr.astype(np.int32), order.astype(np.int32))
         for n in np.unique(ns):
             n = int(n)
             for route in ("fast", "iso", "general", "lindblad"):
@@ -377,13 +403,13 @@ class SpinEngine:
                 g.cost = float(idx.size) * float(n) ** 3
                 g.cs = min(cs, idx.size)
                 g.idx = idx
-                g.d_idx = self._dev(idx.astype(np.int64), torch.int64)
-                g.q = self._dev(batch.q[idx])
-                g.B = self._dev(batch.B[idx])
-                g.Bint = self._dev(batch.Bint[idx])
-                g.p = self._dev(batch.p[idx])
-                g.w = self._dev(batch.w[idx])
-                g.sid = self._dev(batch.sys_id[idx].astype(np.int32), torch.int32)
+                uniq, local = np.unique(sid[idx], return_inverse=True)
+                (g.d_idx, g.q, g.B, g.Bint, g.p, g.w, g.sid, g.sid_local, g.base_ids,
+                 base_sys) = self._upload(
+                    idx.astype(np.int64), *(np.asarray(a[idx], dtype=float) for a in
+                                            (batch.q, batch.B, batch.Bint, batch.p, batch.w)),
+                    sid[idx].astype(np.int32), local.astype(np.int32),
+                    np.arange(uniq.size, dtype=np.int32), sysarr[uniq])
                 g.F = None
                 if route == "general":
                     g.F = self._dev(rho0_factors_host(systems, batch, idx, Br_h), torch.complex128)
@@ -399,23 +425,15 @@ class SpinEngine:
                     s0 = systems[int(batch.sys_id[idx[0]])]
                     g.d_other = n // s0.dims[s0.muon_index]
                 g.mu_half = all(systems[int(k)].dims[systems[int(k)].muon_index] == 2
-                                for k in np.unique(batch.sys_id[idx]))
+                                for k in uniq)
                 # systems shared by many instances get their field-independent
                 # H_sys built once per execute; H = H_sys + Zeeman per instance
-                uniq, local = np.unique(batch.sys_id[idx], return_inverse=True)
                 g.base = None
                 if idx.size >= 2 * uniq.size and uniq.size * n * n * 16 <= self.base_bytes:
                     g.base = torch.empty((uniq.size, n, n), dtype=torch.complex128, device=self.device)
-                    g.base_sys = self._bytes_view(sysarr[uniq])
-                    g.base_ids = self._dev(np.arange(uniq.size, dtype=np.int32), torch.int32)
-                    g.sid_local = self._dev(local.astype(np.int32), torch.int32)
+                    g.base_sys = base_sys
                 self._alloc(g)
                 plan.groups.append(g)
-        order = np.argsort(batch.slot, kind="stable")
-        counts = np.bincount(batch.slot, minlength=batch.n_slots)
-        ptr = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
-        plan.d_ptr = self._dev(ptr, torch.int32)
-        plan.d_order = self._dev(order.astype(np.int32), torch.int32)
         return plan
 
     def _alloc(self, g):
