@@ -96,6 +96,9 @@ hipError_t launch_tridiag(int n, int batch, double *H, double *E, double *work, 
 // Register-resident reduction (matrix in VGPRs, one workgroup per matrix) for
 // n <= 256, same outputs as the panel kernel.
 hipError_t launch_tridiag_rt(int n, int batch, double *H, double *E, double *work, hipStream_t s);
+// Each matrix spread over many workgroups, two launches per column (256 < n <=
+// 1024), same outputs.
+hipError_t launch_tridiag_wide(int n, int batch, double *H, double *E, double *work, hipStream_t s);
 // U = Q Z on MFMA.  off: rows between a reflector's column and its unit
 // element (1 for the one-stage reduction, 16 for the band stage's panels);
 // nref reflectors; zc: start from the complex Z' = Q2 Z of the two-stage

@@ -449,11 +449,18 @@ hipError_t lp_launch(int n, int batch, double *H, double *E, double *work, hipSt
 }  // namespace
 
 // Householder tridiagonalisation for n <= 1024 (hipErrorNotSupported above):
-// the register-resident kernel where the matrix fits one CU's registers, the
-// lower-triangle panel kernel above (panels in the workspace from n = 513 on).
+// the register-resident kernel where the matrix fits one CU's registers; above,
+// the launches that spread each matrix over the chip while there are too few
+// matrices to fill it, else the lower-triangle panel kernel (panels in the
+// workspace from n = 513 on).  The line between the two, in ms spread / one
+// workgroup each: n = 264 at 16 matrices 3.41 / 3.68, at 64 4.26 / 3.78; n = 384
+// at 64 7.14 / 8.52, at 128 9.70 / 8.74; n = 512 at 64 12.0 / 16.5, at 128 18.0 /
+// 18.2; n = 768 at 128 51 / 63, at 192 76 / 72; n = 1024 at 192 157 / 162.
 hipError_t launch_tridiag(int n, int batch, double *H, double *E, double *work, hipStream_t s)
 {
     if (n <= 256) return launch_tridiag_rt(n, batch, H, E, work, s);
+    if (n <= 1024 && batch <= 192 && 4 * batch <= n - 128)
+        return launch_tridiag_wide(n, batch, H, E, work, s);
     if (n <= 512) return lp_launch<MSP_TD_WL, 4, 8, 4>(n, batch, H, E, work, s);
     if (n <= 1024) return lp_launch<MSP_TD_WL, MSP_TD_NBL, 16, MSP_TD_RB1024, true>(n, batch, H, E, work, s);
     return hipErrorNotSupported;

@@ -68,3 +68,14 @@ def test_structured(eng, n):
 def test_batch_rule(eng, n, batch):
     rng = np.random.default_rng(n + batch)
     _check(eng, np.array([_herm(rng, n) for _ in range(batch)]))
+
+
+@pytest.mark.parametrize("n", [257, 264, 265, 319, 320, 321, 384, 511, 513, 700, 1023, 1024])
+def test_few_large(eng, n):
+    rng = np.random.default_rng(n)
+    v = rng.normal(size=n) + 1j * rng.normal(size=n)
+    half = np.zeros((n, n), dtype=complex)
+    m = n // 2
+    half[:m, :m], half[m:, m:] = _herm(rng, m), _herm(rng, n - m)
+    for Hs in ([_herm(rng, n)], [half, np.diag(rng.normal(size=n)) + 0j, np.outer(v, v.conj())]):
+        _check(eng, np.array(Hs))
