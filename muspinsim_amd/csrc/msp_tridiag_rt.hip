@@ -31,8 +31,8 @@
 // 5.2 TB/s past L2); here the matrix is read once.  ms per 4096 matrices, panel
 // kernel (below n = 65: registers in 64-column slots) against this one:
 //   n = 192 18.6 / 10.3, 144 10.7 / 6.6, 128 8.3 / 3.2, 108 6.2 / 2.5,
-//   96 5.1 / 1.7, 72 3.3 / 1.1, 64 2.25 / 0.74, 48 1.82 / 0.37, 32 0.91 / 0.19,
-//   16 0.47 / 0.06; one matrix: n = 192 1.88 / 0.62, 64 0.18 / 0.11; n = 256
+//   96 5.1 / 1.7, 72 3.3 / 1.1, 64 2.25 / 0.74, 48 1.82 / 0.37, 32 0.91 / 0.19;
+//   one matrix: n = 192 1.88 / 0.62, 64 0.18 / 0.11; n = 256
 //   3.3 / 1.65, and for 256 matrices 3.7 / 2.3.
 // Measured and not taken: 16 x 16 tiles in MFMA accumulators dealt to the waves
 // with the rank-2 update on MFMA (n = 192 14.6 ms: FP64 MFMA and FP64 VALU
@@ -501,7 +501,7 @@ hipError_t rt_launch(int n, int batch, double *H, double *E, double *work, hipSt
 
 }  // namespace
 
-// Waves and strips by n: one wave per 16 rows of small matrices, so that many
+// Waves and strips by n (n <= 16 has an eigensolver of its own): few waves for small matrices, so that many
 // matrices share a CU, four waves where two or more workgroups still fit its
 // registers (n <= 128), eight above.  Strips of 4 W rows cover n closely: a
 // strip too many costs 10 to 20 %.
@@ -515,8 +515,6 @@ hipError_t rt_launch(int n, int batch, double *H, double *E, double *work, hipSt
 hipError_t launch_tridiag_rt(int n, int batch, double *H, double *E, double *work, hipStream_t s)
 {
     const bool many = batch > 512;
-    if (n <= 12) return rt_launch<1, 3, 4>(n, batch, H, E, work, s);
-    if (n <= 16) return rt_launch<1, 4, 4>(n, batch, H, E, work, s);
     if (n <= 24) return rt_launch<2, 3, 4>(n, batch, H, E, work, s);
     if (n <= 32) return rt_launch<2, 4, 4>(n, batch, H, E, work, s);
     if (n <= 48 && many) return rt_launch<2, 6, 4>(n, batch, H, E, work, s);
