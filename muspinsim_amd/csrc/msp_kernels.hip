@@ -1324,6 +1324,14 @@ hipError_t launch_timesum(int n, int batch, int ntimes, const double *E, const d
                           int real_mode, const double *times, const double *w, int out_complex,
                           double *out, hipStream_t s)
 {
+    // one wave per 16 times up to n = 112, and up to n = 256 while the waves are
+    // fewer than the SIMDs (each then reads C for itself: with more of them the
+    // kernel below, which shares it between 64 times, is ahead).  Complex C, ms
+    // here / below: n = 108, 1024 x 2000 times 6.9 / 7.7; n = 128 12.5 / 9.5 and
+    // 1 x 1000 0.067 / 0.103; n = 256, 1 x 1000 0.23 / 0.38, 100 x 1000 3.3 / 2.0
+    const size_t waves = cdiv(ntimes, 16) * (size_t)batch;
+    if ((n <= 112 && waves < (size_t)1 << 31) || (n <= 256 && waves <= 1024))
+        return launch_timesum_wave(n, batch, ntimes, E, C, real_mode, times, w, out_complex, out, s);
     dim3 grid(cdiv(ntimes, 64), batch);
     if (real_mode)
         { ProfScope ps_("k_timesum", s);

@@ -316,6 +316,106 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
     }
 }
 
+// ---------------------------------------------------------------------------
+// Time sum of one instance at 16 times by one wave, real or complex C, no
+// workspace: F_j(t) = exp(i phi_j(t)) goes to LDS once per (j, t) (phases formed
+// exactly as k_timesum forms them), Y = C F on FP64 MFMA one 16-row tile at a
+// time with the rows of C read in place (the next k-steps' loads in flight), and
+// P(t) = sum_i conj(F_i) Y_i from the accumulators.
+// Bound by the sines and cosines up to about n = 32 and by the rows of C, which
+// every wave reads from L2, above.  ms for 1024 instances x 2000 times, complex
+// C, 64-row blocks on the VALU (k_timesum) -> here: n = 4 0.72 -> 0.08, 16 0.78
+// -> 0.20, 32 1.33 -> 0.54, 72 5.4 -> 2.7.  Two or four waves in a workgroup, to
+// share C through L1, were 5 to 30 % slower at 1024 instances.
+constexpr int kPF = 4;             // k-steps of C in flight
+template <bool REAL>
+__global__ void __launch_bounds__(64) k_timesum_wave(int n, int ntimes, const double *E,
+                                                     const double *C, const double *times,
+                                                     const double *w, int out_complex, double *out)
+{
+    extern __shared__ double ph[];                // (n padded to 4) x 16 cosines, then sines
+    int tt, b;
+    msp_xcd_tile(gridDim.x, gridDim.y, tt, b);    // an instance's time tiles share one L2
+    const int lane = threadIdx.x, li = lane & 15, lq = lane >> 4;
+    const int nk = (n + 3) / 4;
+    double *pc = ph, *ps = ph + 64 * nk;
+    const double *Eb = E + (size_t)b * n;
+    const double Ec = 0.5 * (Eb[0] + Eb[n - 1]);
+    const int t = 16 * tt + li;
+    const double tl = t < ntimes ? times[t] : 0.0;
+    for (int h = 0; h < nk; ++h) {
+        const int j = 4 * h + lq;
+        double c = 0.0, s = 0.0;
+        if (j < n && t < ntimes) {
+            const double phi = 6.283185307179586 * (Eb[j] - Ec) * tl;
+            sincos(phi, &s, &c);
+        }
+        pc[64 * h + lane] = c;
+        ps[64 * h + lane] = s;
+    }
+    __syncthreads();
+    double Pr = 0.0, Pi = 0.0;
+    for (int i0 = 0; i0 < n; i0 += 16) {
+        const int i = i0 + li;
+        const size_t row = ((size_t)b * n + (i < n ? i : n - 1)) * n;
+        auto load = [&](int h, double &re, double &im) {
+            const int j = 4 * h + lq;
+            const bool ok = i < n && j < n;
+            const int jc = j < n ? j : n - 1;
+            if (REAL) {
+                re = C[row + jc];
+                im = 0.0;
+            } else {
+                re = C[2 * (row + jc)];
+                im = C[2 * (row + jc) + 1];
+            }
+            re = ok ? re : 0.0;
+            im = ok ? im : 0.0;
+        };
+        double ar[kPF], ai[kPF];
+#pragma unroll
+        for (int u = 0; u < kPF; ++u) load(u < nk ? u : nk - 1, ar[u], ai[u]);
+        msp_d4 yr = d4zero(), yi = d4zero();
+        for (int h0 = 0; h0 < nk; h0 += kPF) {
+#pragma unroll
+            for (int u = 0; u < kPF; ++u) {
+                const int h = h0 + u;
+                if (h >= nk) break;
+                const double c = pc[64 * h + lane], s = ps[64 * h + lane];
+                const double xr = ar[u], xi = ai[u];
+                load(h + kPF < nk ? h + kPF : nk - 1, ar[u], ai[u]);
+                yr = mfma_f64(xr, c, yr);
+                yi = mfma_f64(xr, s, yi);
+                if (!REAL) {
+                    yr = mfma_f64(-xi, s, yr);
+                    yi = mfma_f64(xi, c, yi);
+                }
+            }
+        }
+        // slot r is Y[i0 + 4 r + lq][t]
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int h = i0 / 4 + r;
+            if (h >= nk) break;
+            const double c = pc[64 * h + lane], s = ps[64 * h + lane];
+            Pr += c * yr[r] + s * yi[r];
+            Pi += c * yi[r] - s * yr[r];
+        }
+    }
+    Pr += __shfl_xor(Pr, 16, 64);
+    Pr += __shfl_xor(Pr, 32, 64);
+    Pi += __shfl_xor(Pi, 16, 64);
+    Pi += __shfl_xor(Pi, 32, 64);
+    if (lq == 0 && t < ntimes) {
+        if (out_complex) {
+            out[2 * ((size_t)b * ntimes + t)] = Pr;
+            out[2 * ((size_t)b * ntimes + t) + 1] = Pi;
+        } else {
+            out[(size_t)b * ntimes + t] = (w ? w[b] : 1.0) * Pr;
+        }
+    }
+}
+
 }  // namespace
 
 int timesum_mfma_ldt(int ntimes) { return (ntimes + kTT - 1) / kTT * kTT; }
@@ -352,10 +452,32 @@ size_t timesum_mfma64_workspace(int n, int batch, int ntimes)
     return (size_t)2 * n * timesum_mfma_ldt(ntimes) * sizeof(double) * (size_t)batch;
 }
 
+// n <= 256 (256 bytes of LDS per dimension and wave).
+hipError_t launch_timesum_wave(int n, int batch, int ntimes, const double *E, const double *C,
+                               int real_mode, const double *times, const double *w, int out_complex,
+                               double *out, hipStream_t s)
+{
+    const size_t lds = (size_t)1024 * ((n + 3) / 4);
+    const dim3 grid((ntimes + 15) / 16, batch);
+    ProfScope ps_("k_timesum", s);
+    if (real_mode)
+        hipLaunchKernelGGL(k_timesum_wave<true>, grid, dim3(64), lds, s, n, ntimes, E, C, times, w,
+                           out_complex, out);
+    else
+        hipLaunchKernelGGL(k_timesum_wave<false>, grid, dim3(64), lds, s, n, ntimes, E, C, times, w,
+                           out_complex, out);
+    return hipGetLastError();
+}
+
 hipError_t launch_timesum_mfma64(int n, int batch, int ntimes, const double *E, const double *C,
                                  const double *times, const double *w, double *out, void *work,
                                  hipStream_t s)
 {
+    // up to n = 48 the whole sum in one wave per 16 times is ahead of a table
+    // and 64-row tiles: ms for 1024 x 2000 times n = 16 0.17 / 0.47, 32 0.43 /
+    // 0.77, 48 0.83 / 1.12, 64 1.45 / 1.49; 100 x 1000 n = 48 0.061 / 0.071, 64
+    // 0.094 / 0.085
+    if (n <= 48) return launch_timesum_wave(n, batch, ntimes, E, C, 1, times, w, 0, out, s);
     const int ldt = timesum_mfma_ldt(ntimes);
     double *Fc = (double *)work;
     double *Fs = Fc + (size_t)n * ldt * batch;

@@ -105,3 +105,33 @@ def test_engine_timesum_paths_vs_oracle(gpu_lib, precision, cfg):
     ref = opipe.run(systems, batch)
     err = np.abs(got - ref).max()
     assert err <= (1e-6 if precision == "mixed" else 1e-10), f"max |dP| = {err:.3e}"
+
+
+@pytest.mark.parametrize("n,T,batch", [(1, 1, 2), (3, 15, 9), (4, 16, 1), (5, 17, 3), (15, 33, 2),
+                                       (16, 40, 11), (17, 16, 3), (48, 31, 2), (63, 65, 8),
+                                       (65, 47, 3), (112, 33, 2), (113, 1, 1), (200, 64, 1),
+                                       (255, 20, 3), (256, 33, 1)])
+@pytest.mark.parametrize("real", [0, 1])
+def test_timesum_one_wave(gpu_lib, n, T, batch, real):
+    """msp_timesum's one-wave form, with both kinds of C and of output, a C that
+    is neither symmetric nor Hermitian, and every tail of its 16 x 16 x 4 steps."""
+    from muspinsim_amd import _native as N
+    rng = np.random.default_rng(1000 * n + T + real)
+    E, _, t, w = _timesum_inputs(rng, n, batch, T, spread=100.0)
+    C = rng.normal(size=(batch, n, n)) + 0j
+    if not real:
+        C = C + 1j * rng.normal(size=(batch, n, n))
+    dE, dt, dw = (_dev(x) for x in (E, t, w))
+    dC = _dev(C.real) if real else _dev(C, torch.complex128)
+    st = torch.cuda.current_stream().cuda_stream
+    F = np.exp(2j * np.pi * (E - 0.5 * (E[:, :1] + E[:, -1:]))[:, :, None] * t)
+    ref = (np.conj(F) * (C @ F)).sum(1)
+    for cplx in (0, 1):
+        out = torch.full((batch, T), np.nan, device="cuda",
+                         dtype=torch.complex128 if cplx else torch.float64)
+        N.check(gpu_lib.msp_timesum(n, batch, T, dE.data_ptr(), dC.data_ptr(), real, dt.data_ptr(),
+                                    None if cplx else dw.data_ptr(), cplx, out.data_ptr(), st))
+        want = ref if cplx else w[:, None] * ref.real
+        phmax = 2 * np.pi * (E.max() - E.min()) * t.max()
+        assert np.abs(out.cpu().numpy() - want).max() <= (
+            4e-16 * max(phmax, 10.0) * 2.0 * np.abs(C).sum((1, 2)).max())
