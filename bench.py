@@ -38,7 +38,7 @@ def algorithmic(kernel, n, ntimes, real_mode=True):
         return "flop", 8.0 * n ** 3
     if kernel == "k_gemm_cn":
         return "flop", 8.0 * n ** 3
-    if kernel == "k_eigh_jacobi":
+    if kernel in ("k_eigh_jacobi", "k_eigh_small"):
         return "flop", (16.0 / 3.0 + 8.0) * n ** 3
     if kernel == "k_lindblad_modes":
         # Liouvillian order N = n^2: Hessenberg + Schur + eigenvectors (LAPACK's

@@ -94,9 +94,11 @@ typedef struct MspTerm {
 } MspTerm;
 
 /* Eigensolver selection for msp_eigh. */
-#define MSP_EIGH_AUTO 0
+#define MSP_EIGH_AUTO 0     /* n <= 16: the one-wave Jacobi kernel of MSP_EIGH_DC; n <= 64:
+                               MSP_EIGH_JACOBI; above: MSP_EIGH_DC */
 #define MSP_EIGH_JACOBI 1   /* LDS-resident cyclic Jacobi, n <= 64 */
-#define MSP_EIGH_DC 2       /* Householder + divide and conquer, any n */
+#define MSP_EIGH_DC 2       /* one-wave Jacobi up to n = 16, Householder + divide and conquer
+                               above, any n */
 #define MSP_EIGH_DC2 3      /* two-stage reduction (band of 16 on FP64 matrix cores,
                                then bulge chasing) + divide and conquer, 34 <= n <= 256 */
 

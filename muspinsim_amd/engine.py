@@ -4,7 +4,7 @@ One call of :meth:`SpinEngine.run` carries a whole set of instances
 (orientation x field x temperature snapshots) through
 
   (a) msp_rotate_fields + msp_build_h   B' = q.B + B_int, H = H_sys + Zeeman(B')
-  (b) msp_eigh                          Jacobi in LDS (n <= 64) or Householder + D&C
+  (b) msp_eigh                          one-wave Jacobi (n <= 16) or Householder + D&C
   (c) msp_apply_muon_op + msp_gemm_cn   O' = U^H (p'.S_mu) U   (and rho' when needed)
   (d) msp_form_c + msp_timesum / msp_integral, then msp_accumulate
       (weights, 1/avg_N and the results array, in instance order)
