@@ -114,6 +114,9 @@ __global__ void __launch_bounds__(64) k_eigh_small(int n, int batch, const doubl
     for (int o = M * M / 2; o > 0; o >>= 1) fro += __shfl_xor(fro, o, 64);
     // pair elements at or below 2^-53 ||A||_F are left alone
     const double skip = fro * 0x1p-106;
+    // a NaN or infinite entry: no rotation is made (every comparison with skip is
+    // false); info = 1 and NaN results below
+    const bool bad = !(fro < INFINITY);
     const int i = l / M, j = l - i * M;
     const bool on = i < m && j < m;
     wave_sync();
@@ -184,9 +187,9 @@ __global__ void __launch_bounds__(64) k_eigh_small(int n, int batch, const doubl
         for (int o = M * M / 2; o > 0; o >>= 1) off = fmax(off, __shfl_xor(off, o, 64));
         st = off <= skip ? 0 : 1;
     }
-    if (l == 0 && real_one) info[b] = st;
+    if (l == 0 && real_one) info[b] = bad ? 1 : st;
 
-    // ascending order
+    // ascending order (a NaN diagonal has none)
     for (int r = l; r < n; r += M * M) {
         const double d = A[r * LD + r].re;
         int rank = 0;
@@ -194,15 +197,16 @@ __global__ void __launch_bounds__(64) k_eigh_small(int n, int batch, const doubl
             const double dk = A[k * LD + k].re;
             rank += (dk < d || (dk == d && k < r)) ? 1 : 0;
         }
+        if (bad) rank = r;
         order[sub][rank] = r;
-        if (real_one) E[(size_t)b * n + rank] = ldexp(d, ex);
+        if (real_one) E[(size_t)b * n + rank] = bad ? NAN : ldexp(d, ex);
     }
     wave_sync();
     if (!real_one) return;
     cdbl *Ub = (cdbl *)U + (size_t)b * n * n;
     for (int x = l; x < n * n; x += M * M) {
         const int r = x / n, k = x - r * n;
-        Ub[x] = V[r * LD + order[sub][k]];
+        Ub[x] = bad ? cmk(NAN, NAN) : V[r * LD + order[sub][k]];
     }
 }
 

@@ -79,3 +79,27 @@ def test_few_large(eng, n):
     half[:m, :m], half[m:, m:] = _herm(rng, m), _herm(rng, n - m)
     for Hs in ([_herm(rng, n)], [half, np.diag(rng.normal(size=n)) + 0j, np.outer(v, v.conj())]):
         _check(eng, np.array(Hs))
+
+
+@pytest.mark.parametrize("n", [1, 2, 4, 5, 8, 9, 16])
+def test_small_non_finite(eng, n):
+    """n <= 16: a matrix with a NaN or infinite entry reports info != 0 with NaN
+    eigenvalues and vectors; the matrices that share its wave are unaffected."""
+    from muspinsim_amd import _native as N
+    rng = np.random.default_rng(n)
+    good = np.array([_herm(rng, n) for _ in range(16)])
+    Hs = good.copy()
+    bad = {1: (n - 1, 0, np.nan), 4: (0, 0, np.nan), 6: (n - 1, n - 1, np.inf),
+           9: (n - 1, 0, -np.inf), 15: (n // 2, 0, complex(0.0 if n > 1 else np.nan, np.nan))}
+    for k, (i, j, x) in bad.items():
+        Hs[k, i, j] = x
+    for method in (N.MSP_EIGH_DC, N.MSP_EIGH_AUTO):
+        E0, U0, _ = eng.eigh(torch.as_tensor(good).cuda(), method=method)
+        E, U, info = eng.eigh(torch.as_tensor(Hs).cuda(), method=method)
+        for k in range(len(Hs)):
+            if k in bad:
+                assert int(info[k]) != 0
+                assert torch.isnan(E[k]).all() and torch.isnan(torch.view_as_real(U[k])).all()
+            else:
+                assert int(info[k]) == 0
+                assert torch.equal(E[k], E0[k]) and torch.equal(U[k], U0[k])
