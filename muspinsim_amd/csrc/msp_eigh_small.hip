@@ -29,13 +29,17 @@
 
 namespace {
 
-// 1/sqrt(t), hardware estimate and two Newton steps
+// 1/sqrt(t): hardware estimate and two Newton steps, each adding a small
+// correction to y.  The product y (1.5 - t y^2 / 2) of the same length rounds its
+// factor near one instead and is biased: at n = 16 the squared norms of the
+// vectors were off by -2.2e-15 on average (+6e-16 so, LDS Jacobi +1.6e-15), the
+// eigenvalues by 3.7e-16 ||H|| rms (2.1e-16 so, LDS Jacobi 2.0e-16).
 __device__ inline double small_rsqrt(double t)
 {
     double y = __builtin_amdgcn_rsq(t);
     const double h = 0.5 * t;
-    y = y * fma(-h * y, y, 1.5);
-    return y * fma(-h * y, y, 1.5);
+    y = fma(y, fma(-h * y, y, 0.5), y);
+    return fma(y, fma(-h * y, y, 0.5), y);
 }
 
 // a wave executes LDS operations in order: the compiler must keep them so

@@ -103,3 +103,18 @@ def test_small_non_finite(eng, n):
             else:
                 assert int(info[k]) == 0
                 assert torch.equal(E[k], E0[k]) and torch.equal(U[k], U0[k])
+
+
+@pytest.mark.parametrize("n,sweeps", [(8, 7), (12, 8), (16, 8)])
+def test_small_norms(eng, n, sweeps):
+    """Rotations of the n <= 16 solver are unit to within rounding: a vector goes
+    through n - 1 of them per sweep, so its squared norm is off by at most about
+    eps / 2 times the root of their number (rms; a biased rotation adds up to
+    their number instead, twice as much here)."""
+    from muspinsim_amd import _native as N
+    rng = np.random.default_rng(n)
+    X = rng.normal(size=(4000, n, n)) + 1j * rng.normal(size=(4000, n, n))
+    _, U, _ = eng.eigh(torch.as_tensor(X + X.conj().swapaxes(1, 2)).cuda(), method=N.MSP_EIGH_DC)
+    U = U.cpu().numpy()
+    off = (U.real.astype(np.longdouble) ** 2 + U.imag.astype(np.longdouble) ** 2).sum(1) - 1
+    assert np.sqrt(float((off ** 2).mean())) <= 1.4 * 2.0 ** -53 * np.sqrt(sweeps * (n - 1))
