@@ -215,6 +215,9 @@ MSP_HD double ns_recip(double x)
     return fma(r, e, r);
 #endif
 }
+// (Each Newton step adds a small correction to y: the product y (1.5 - x y^2 / 2)
+// is biased, and thousands of rotations scaled by it moved the eigenvalues of a
+// 64 x 64 matrix by 3.7e-15 ||A|| rms, against 1.1e-15.)
 MSP_HD double ns_rsqrt(double x)
 {
 #ifdef MSP_HOST_BUILD
@@ -222,8 +225,8 @@ MSP_HD double ns_rsqrt(double x)
 #else
     double y = __builtin_amdgcn_rsq(x);
     const double h = 0.5 * x;
-    y = y * fma(-h * y, y, 1.5);
-    y = y * fma(-h * y, y, 1.5);
+    y = fma(y, fma(-h * y, y, 0.5), y);
+    y = fma(y, fma(-h * y, y, 0.5), y);
     return y;
 #endif
 }

@@ -63,3 +63,22 @@ def test_zero_matrix_and_no_operators(eng):
     r = np.ones((1, N))
     lam, _, c, _ = eng.lindblad_modes(_dev(np.zeros((1, N, N))), _dev(r), None, want_c=True)
     assert np.all(lam.cpu().numpy() == 0) and np.allclose(c.cpu().numpy(), r)
+
+
+@pytest.mark.parametrize("N", [9, 16, 36, 64])
+def test_eigenvalue_rounding(eng, N):
+    """Rotations of the QR sweeps are unit to within rounding: an eigenvalue of a
+    normal matrix goes through two per sweep and about 2.5 N sweeps, so it is off
+    by about eps / 2 times the root of their number (rms, relative to the norm;
+    biased rotations add up to their number instead)."""
+    rng = np.random.default_rng(N)
+    G = rng.normal(size=(200, N, N)) + 1j * rng.normal(size=(200, N, N))
+    G = G + np.conj(np.swapaxes(G, 1, 2))
+    one = np.ones((200, N))
+    lam, _, _, _ = eng.lindblad_modes(_dev(1j * G), _dev(one), _dev(one[:, None]))
+    lam = lam.cpu().numpy()
+    ref = np.linalg.eigvalsh(G)
+    scale = np.abs(ref).max(1, keepdims=True)
+    err = np.sqrt((((np.sort(lam.imag, 1) - ref) / scale) ** 2).mean())
+    assert err <= 2.0 ** -53 * np.sqrt(2 * 2.5 * N)
+    assert np.sqrt(((lam.real / scale) ** 2).mean()) <= 2.0 ** -53 * np.sqrt(2 * 2.5 * N)
