@@ -173,17 +173,32 @@ __device__ inline bool digits_packable(const MspSystem &S)
     return ok;
 }
 
-// H[b][a][c]: the system's terms (or a precomputed base) + Zeeman, ept elements
-// per thread.  With the digits packed in LDS, one XOR tells an element whose row
-// and column differ in three spins or more (zero, or the base: all but a few per
-// row of a large system) and which spins differ in the others; systems with a
-// multiplicity above 16 take the per-element path.  Bound by the term loop of
-// the elements that are left.  4096 instances of n = 4 .. 1024: 10.7 ms with
-// digits by division for every element (their arrays in scratch), 7.2 here.
+// H[b][a][c]: the system's terms (or a precomputed base) + Zeeman, one thread
+// per element, index digits by division (any multiplicities).
 __global__ void __launch_bounds__(256) k_build_h(int n, const MspSystem *systems,
                                                  const MspTerm *terms, const int32_t *sys_id,
                                                  const double *Br, const double *base, int zeeman,
-                                                 int lower, int ept, double *H)
+                                                 int lower, double *H)
+{
+    const int b = blockIdx.y;
+    const int idx = blockIdx.x * 256 + threadIdx.x;
+    if (idx >= n * n) return;
+    if (lower && idx % n > idx / n) return;
+    const int s = sys_id ? sys_id[b] : 0;
+    const cdbl *bm = base ? (const cdbl *)base + (size_t)s * n * n : nullptr;
+    ((cdbl *)H)[(size_t)b * n * n + idx] = h_element(n, systems[s], terms, bm, Br + 3 * b, zeeman, idx);
+}
+
+// The same for large n, ept elements per thread.  With the digits packed in LDS,
+// one XOR tells an element whose row and column differ in three spins or more
+// (zero, or the base: all but a few per row of a large system) and which spins
+// differ in the others; systems with a multiplicity above 16 take the
+// per-element path.  Bound by the term loop of the elements that are left.
+__global__ void __launch_bounds__(256) k_build_h_packed(int n, const MspSystem *systems,
+                                                        const MspTerm *terms,
+                                                        const int32_t *sys_id, const double *Br,
+                                                        const double *base, int zeeman, int lower,
+                                                        int ept, double *H)
 {
     extern __shared__ unsigned long long digs[];
     struct Digit {
@@ -1058,14 +1073,23 @@ hipError_t launch_build_h(int n, int batch, const MspSystem *systems, const MspT
         hipLaunchKernelGGL(k_build_h_base, dim3(cdiv(cnt, 256 * kBuildEPT), batch),
                            dim3(256), sizeof(unsigned long long) * n, s, n, systems, terms, sys_id,
                            Br, base, lower, H);
-    } else {
-        // a thread takes several elements (up to 16, sharing one digit table)
-        // once the launch still fills the chip with 2048 workgroups
-        const size_t wgs = cdiv((size_t)n * n, 256);
-        const int ept = (int)std::min<size_t>(16, std::max<size_t>(1, wgs * batch / 2048));
-        hipLaunchKernelGGL(k_build_h, dim3(cdiv(wgs, ept), batch), dim3(256),
+        return hipGetLastError();
+    }
+    // A thread of the packed form takes up to 16 elements, sharing one digit
+    // table, while 8192 workgroups are left.  It pays from about four on and
+    // above n = 256; with fewer elements the slowest wave's term loop decides, or
+    // too few elements are skipped.  us an element per thread / packed, lower
+    // triangles: n = 288, 80 matrices 365 / 380, 300 1295 / 900; n = 2048, one 365
+    // / 385, six 2300 / 1460; n = 256, 300 2340 / 2560
+    const size_t wgs = cdiv((size_t)n * n, 256);
+    if (n > 256 && wgs * batch >= 4 * 8192) {
+        const int ept = (int)std::min<size_t>(16, wgs * batch / 8192);
+        hipLaunchKernelGGL(k_build_h_packed, dim3(cdiv(wgs, ept), batch), dim3(256),
                            sizeof(unsigned long long) * n, s, n, systems, terms, sys_id, Br, base,
                            zeeman, lower, ept, H);
+    } else {
+        hipLaunchKernelGGL(k_build_h, dim3(wgs, batch), dim3(256), 0, s, n, systems, terms, sys_id,
+                           Br, base, zeeman, lower, H);
     }
     return hipGetLastError();
 }

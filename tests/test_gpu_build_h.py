@@ -1,6 +1,7 @@
-"""Hamiltonian build from the terms against the oracle: one and several elements
-per thread (few and many instances), spin digits up to the packed limit of 15 and
-above it, full matrices and lower triangles."""
+"""Hamiltonian build from the terms against the oracle: an element per thread, and
+with packed spin digits several (n > 256 and many elements: both sides of that
+rule), digits up to the packed limit of 15 and above it, full matrices and lower
+triangles."""
 
 import numpy as np
 import pytest
@@ -14,7 +15,10 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("lower", [False, True])
 @pytest.mark.parametrize("Is,nb", [([0.5], 1), ([0.5, 1.0, 0.5], 5000), ([0.5] * 8, 3),
                                    ([0.5] * 8, 40), ([0.5, 3.5, 0.5, 1.0], 70), ([7.5, 0.5], 600),
-                                   ([0.5, 8.5], 600)])
+                                   ([0.5, 8.5], 600),
+                                   # from 32,768 workgroups of 256 elements on
+                                   ([0.5, 1.0, 1.0, 2.5, 1.0], 79), ([0.5, 1.0, 1.0, 2.5, 1.0], 80),
+                                   ([0.5, 8.5, 3.5], 102), ([0.5] * 9, 31), ([0.5] * 9, 32)])
 def test_from_terms(gpu_lib, Is, nb, lower):
     from muspinsim_amd import _native as N
     from muspinsim_amd.engine import SpinEngine, SystemDesc, pack_systems
