@@ -22,6 +22,8 @@ namespace {
 constexpr int kTile = 64;        // (j, k) tile edge
 constexpr int kTC = 8;           // times per chunk
 constexpr int kLd = kTile + 16;  // row stride of the LDS phases (two rows cover all banks)
+constexpr int kPairs = 16;       // k_adjoint_freq_pairs: (j, k) tile edge
+constexpr int kPairTimes = 64;   // and times per chunk
 
 // R and S of one 64 x 64 tile (j0 <= k0) of one instance, and of its mirror
 // (R symmetric, S antisymmetric): with w_jk = w_j - w_k both are sums over times
@@ -143,6 +145,60 @@ __global__ void __launch_bounds__(512) k_adjoint_freq(int n, int ntimes, const d
     }
 }
 
+// The same by one thread per (j, k), a workgroup per 16 x 16 tile: for few
+// instances, over which the tiles above would leave most CUs idle.
+__global__ void __launch_bounds__(256) k_adjoint_freq_pairs(int n, int ntimes, const double *E,
+                                                            const double *times, const double *r,
+                                                            const int32_t *slot, const double *w,
+                                                            double scale, double *R, double *S)
+{
+    __shared__ cdbl Pj[kPairs][kPairTimes + 1];
+    __shared__ cdbl Pk[kPairs][kPairTimes + 1];
+    __shared__ double rt[kPairTimes], tt[kPairTimes];
+    const int b = blockIdx.z;
+    const int j0 = blockIdx.y * kPairs, k0 = blockIdx.x * kPairs;
+    const int tid = threadIdx.x, jj = tid / kPairs, kk = tid % kPairs;
+    const double *Eb = E + (size_t)b * n;
+    const double Ec = 0.5 * (Eb[0] + Eb[n - 1]);
+    const double *rb = r + (size_t)(slot ? slot[b] : 0) * ntimes;
+    const double twopi = 6.283185307179586;
+    double sr = 0.0, ss = 0.0;
+    for (int t0 = 0; t0 < ntimes; t0 += kPairTimes) {
+        __syncthreads();
+        for (int l = tid; l < kPairTimes; l += 256) {
+            const int t = t0 + l;
+            rt[l] = (t < ntimes) ? rb[t] : 0.0;
+            tt[l] = (t < ntimes) ? times[t] : 0.0;
+        }
+        for (int l = tid; l < 2 * kPairs * kPairTimes; l += 256) {
+            const int which = l / (kPairs * kPairTimes), rem = l % (kPairs * kPairTimes);
+            const int a = rem / kPairTimes, c = rem % kPairTimes;
+            const int t = t0 + c;
+            const int idx = (which ? k0 : j0) + a;
+            double sn = 0.0, cs = 1.0;
+            if (idx < n && t < ntimes) sincos(twopi * (Eb[idx] - Ec) * times[t], &sn, &cs);
+            if (which) Pk[a][c] = cmk(cs, sn);
+            else Pj[a][c] = cmk(cs, sn);
+        }
+        __syncthreads();
+        const int lim = (ntimes - t0 < kPairTimes) ? ntimes - t0 : kPairTimes;
+        for (int c = 0; c < lim; ++c) {
+            // exp(i w_jk t) = Pj conj(Pk)
+            const cdbl pj = Pj[jj][c], pk = Pk[kk][c];
+            const double re = pj.re * pk.re + pj.im * pk.im;
+            const double im = pj.im * pk.re - pj.re * pk.im;
+            sr = fma(rt[c], re, sr);
+            ss = fma(rt[c] * tt[c], im, ss);
+        }
+    }
+    const int j = j0 + jj, k = k0 + kk;
+    if (j < n && k < n) {
+        const double f = scale * (w ? w[b] : 1.0);
+        R[(size_t)b * n * n + (size_t)j * n + k] = f * sr;
+        S[(size_t)b * n * n + (size_t)j * n + k] = f * ss;
+    }
+}
+
 // M = R o O (elementwise, R real, O complex)
 __global__ void k_hadamard_real(int n, int batch, const double *R, const double *O, double *M)
 {
@@ -234,6 +290,21 @@ hipError_t launch_adjoint_freq(int n, int batch, int ntimes, const double *E, co
                                double *R, double *S, hipStream_t s)
 {
     ProfScope ps_("k_adjoint_freq", s);
+    // The matrix form has one workgroup per 64 x 64 tile of an instance's upper
+    // triangle, the thread-per-pair form one per 16 x 16 tile of all of it: the
+    // first is ahead once the second's workgroups fill the chip about 4.5 times
+    // over (2.8 times up to n = 48, where it forms fewer phases twice), and never
+    // when n fits one small tile.  ms pairs / matrix form, 1000 times: n = 16, 512
+    // instances 0.12 / 0.19; n = 32, 128 0.091 / 0.090, 256 0.18 / 0.12; n = 64, 48
+    // 0.14 / 0.17, 96 0.28 / 0.18; n = 128, 16 0.21 / 0.24, 24 0.32 / 0.25; n = 256, 4
+    // 0.22 / 0.24, 8 0.41 / 0.25; n = 64, one instance, 4000 times 0.37 / 0.70
+    const unsigned np = cdivu(n, kPairs);
+    const size_t pair_wgs = (size_t)np * np * batch;
+    if (n <= kPairs || pair_wgs <= (n <= 48 ? 720 : 1152)) {
+        hipLaunchKernelGGL(k_adjoint_freq_pairs, dim3(np, np, batch), dim3(256), 0, s, n, ntimes, E,
+                           times, r, slot, w, scale, R, S);
+        return hipGetLastError();
+    }
     const unsigned nt = cdivu(n, kTile);
     hipLaunchKernelGGL(k_adjoint_freq, dim3(nt * (nt + 1) / 2, batch), dim3(512), 0, s, n, ntimes, E, times, r, slot, w,
                        scale, R, S);

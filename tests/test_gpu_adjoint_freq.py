@@ -1,6 +1,7 @@
 """Frequency sums of the adjoint, R_jk = sum_t r cos w_jk t and S_jk = sum_t r t
-sin w_jk t, against numpy at the edges of the kernel's 64 x 64 tiles and 8-time
-chunks."""
+sin w_jk t, against numpy at the edges of the two kernels' tiles (16 x 16 and 64
+times for few instances, 64 x 64 and 8 times for many) and on both sides of the
+rule between them."""
 
 import numpy as np
 import pytest
@@ -11,14 +12,25 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("n,nt", [(1, 5), (3, 1), (15, 8), (16, 9), (17, 16), (48, 17), (63, 40),
                                   (64, 33), (65, 7), (80, 24), (128, 15), (130, 31), (16, 0)])
-def test_frequency_sums(gpu_lib, n, nt):
+@pytest.mark.parametrize("nb", [3, 0])
+def test_frequency_sums(gpu_lib, n, nt, nb):
+    """nb = 0: the smallest batch of the matrix form, and one below it."""
+    if nb == 0 and n > 16:
+        first = (720 if n <= 48 else 1152) // ((n + 15) // 16) ** 2 + 1
+        _compare(gpu_lib, n, nt, first - 1)
+        _compare(gpu_lib, n, nt, first)
+    else:
+        _compare(gpu_lib, n, nt, nb or 700)
+
+
+def _compare(gpu_lib, n, nt, nb):
     from muspinsim_amd import _native as N
     rng = np.random.default_rng(100 * n + nt)
-    nb, slots = 3, 2
+    slots = 2
     E = np.sort(rng.normal(0, 30.0, (nb, n)), axis=1)
     t = rng.uniform(0, 10.0, nt)
     r = rng.normal(size=(slots, nt))
-    slot = np.array([1, 0, 1], dtype=np.int32)
+    slot = (1 - np.arange(nb) % 2).astype(np.int32)
     w = rng.uniform(0.5, 2.0, nb)
     d = [torch.as_tensor(a).cuda() for a in (E, np.append(t, 0.0), np.append(r.ravel(), 0.0), slot, w)]
     R = torch.full((nb, n, n), np.nan, dtype=torch.float64, device="cuda")
