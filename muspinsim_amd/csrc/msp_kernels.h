@@ -79,6 +79,8 @@ hipError_t launch_gemm_cn(int n, int batch, const double *A, const double *B, do
 hipError_t launch_form_c(int n, int batch, const double *rho, const double *obs, int real_mode,
                          double alpha, double beta, double *C, hipStream_t s);
 // One wave per 16 times, FP64 MFMA, no workspace, n <= 256.
+// (timesum_wave_resident: its waves that the chip's LDS holds at once.)
+size_t timesum_wave_resident(int n);
 hipError_t launch_timesum_wave(int n, int batch, int ntimes, const double *E, const double *C,
                                int real_mode, const double *times, const double *w, int out_complex,
                                double *out, hipStream_t s);

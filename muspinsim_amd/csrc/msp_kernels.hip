@@ -1348,13 +1348,17 @@ hipError_t launch_timesum(int n, int batch, int ntimes, const double *E, const d
                           int real_mode, const double *times, const double *w, int out_complex,
                           double *out, hipStream_t s)
 {
-    // one wave per 16 times up to n = 112, and up to n = 256 while the waves are
-    // fewer than the SIMDs (each then reads C for itself: with more of them the
-    // kernel below, which shares it between 64 times, is ahead).  Complex C, ms
-    // here / below: n = 108, 1024 x 2000 times 6.9 / 7.7; n = 128 12.5 / 9.5 and
-    // 1 x 1000 0.067 / 0.103; n = 256, 1 x 1000 0.23 / 0.38, 100 x 1000 3.3 / 2.0
+    // One wave per 16 times up to n = 96 (complex C 104), and up to n = 256 while
+    // all its waves are resident at once: each reads C for itself and keeps its
+    // phases in LDS, and with more of them the kernel below, which shares C
+    // between 64 times, is ahead.  ms here / below: real C, n = 96, 1024 x 50 times
+    // 0.156 / 0.182, n = 108 0.27 / 0.20; complex, n = 104, 4096 x 100 1.73 / 2.14, n
+    // = 108 2.33 / 2.14; n = 108, 64 x 300 0.079 / 0.135; n = 192, 756 waves 0.139 /
+    // 0.221, 1008 waves 0.349 / 0.231; n = 256, 504 waves 0.236 / 0.385, 1008 waves
+    // 0.467 / 0.403
     const size_t waves = cdiv(ntimes, 16) * (size_t)batch;
-    if ((n <= 112 && waves < (size_t)1 << 31) || (n <= 256 && waves <= 1024))
+    if ((n <= (real_mode ? 96 : 104) && waves < (size_t)1 << 31) ||
+        (n <= 256 && waves <= timesum_wave_resident(n)))
         return launch_timesum_wave(n, batch, ntimes, E, C, real_mode, times, w, out_complex, out, s);
     dim3 grid(cdiv(ntimes, 64), batch);
     if (real_mode)

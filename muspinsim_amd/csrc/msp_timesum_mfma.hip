@@ -452,12 +452,18 @@ size_t timesum_mfma64_workspace(int n, int batch, int ntimes)
     return (size_t)2 * n * timesum_mfma_ldt(ntimes) * sizeof(double) * (size_t)batch;
 }
 
+static size_t timesum_wave_lds(int n) { return (size_t)1024 * ((n + 3) / 4); }
+
+// 256 CUs of 160 KB, handed out in pieces of 1280 bytes (one more KB per wave
+// covers the rounding).
+size_t timesum_wave_resident(int n) { return 256 * ((160 << 10) / (timesum_wave_lds(n) + 1024)); }
+
 // n <= 256 (256 bytes of LDS per dimension and wave).
 hipError_t launch_timesum_wave(int n, int batch, int ntimes, const double *E, const double *C,
                                int real_mode, const double *times, const double *w, int out_complex,
                                double *out, hipStream_t s)
 {
-    const size_t lds = (size_t)1024 * ((n + 3) / 4);
+    const size_t lds = timesum_wave_lds(n);
     const dim3 grid((ntimes + 15) / 16, batch);
     ProfScope ps_("k_timesum", s);
     if (real_mode)
@@ -473,11 +479,13 @@ hipError_t launch_timesum_mfma64(int n, int batch, int ntimes, const double *E, 
                                  const double *times, const double *w, double *out, void *work,
                                  hipStream_t s)
 {
-    // up to n = 48 the whole sum in one wave per 16 times is ahead of a table
-    // and 64-row tiles: ms for 1024 x 2000 times n = 16 0.17 / 0.47, 32 0.43 /
-    // 0.77, 48 0.83 / 1.12, 64 1.45 / 1.49; 100 x 1000 n = 48 0.061 / 0.071, 64
-    // 0.094 / 0.085
-    if (n <= 48) return launch_timesum_wave(n, batch, ntimes, E, C, 1, times, w, 0, out, s);
+    // up to n = 48 (40 with too few waves to hide their latency) the whole sum in
+    // one wave per 16 times is ahead of a table and 64-row tiles: ms for 1024 x
+    // 2000 times n = 16 0.17 / 0.47, 32 0.43 / 0.77, 48 0.83 / 1.12, 64 1.45 / 1.49;
+    // 100 x 1000 n = 48 0.061 / 0.071, 64 0.094 / 0.085; 1 x 1000 (63 waves) n = 40
+    // 0.0104 / 0.0109, 48 0.0119 / 0.0110
+    const size_t waves = (size_t)((ntimes + 15) / 16) * batch;
+    if (n <= 40 || (n <= 48 && waves >= 192)) return launch_timesum_wave(n, batch, ntimes, E, C, 1, times, w, 0, out, s);
     const int ldt = timesum_mfma_ldt(ntimes);
     double *Fc = (double *)work;
     double *Fs = Fc + (size_t)n * ldt * batch;

@@ -1,9 +1,10 @@
-"""Time sums of the real routes on matrix cores, on the GPU.
+"""Time sums on the GPU: the one-wave form, the phase-table form on matrix cores
+and the 64-time form on the VALU, and the rules that choose between them.
 
-msp_timesum_mfma64 (FP64 phase table + FP64 MFMA GEMM) forms the same phases
-as msp_timesum with the same expression and differs from it only in the
-order of the FP64 sums: both are held to 1e-13 sum_ij |C_ij| of each other
-and to the numpy sum.  End to end, SpinEngine is forced onto each time-sum
+msp_timesum_mfma64 (FP64 phase table + FP64 MFMA GEMM, or the one-wave form up to
+n = 48) forms the same phases as msp_timesum with the same expression and differs
+from it only in the order of the FP64 sums: both are held to 1e-13 sum_ij |C_ij|
+of each other and to the numpy sum.  End to end, SpinEngine is forced onto each time-sum
 path (thresholds 0) and compared with the FP64 oracle: <= 1e-10 (PARITY) for
 the FP64 paths, <= 1e-6 for the mixed one.
 """
@@ -29,10 +30,14 @@ def _timesum_inputs(rng, n, batch, T, spread=2000.0, tmax=20.0):
 
 
 @pytest.mark.parametrize("n,T,batch", [(1, 5, 2), (16, 64, 3), (33, 70, 11), (64, 200, 4),
-                                       (100, 129, 5), (512, 300, 2)])
+                                       (100, 129, 5), (512, 300, 2),
+                                       # msp_timesum's 64-time VALU form from here on
+                                       (97, 2250, 11), (130, 1130, 18), (192, 1130, 11),
+                                       (257, 65, 9)])
 def test_timesum_mfma64_vs_fp64_valu(gpu_lib, n, T, batch):
-    """FP64 matrix-core time sum against msp_timesum (FP64 VALU) and numpy,
-    including row, column and time tails and phases up to ~1e6 rad."""
+    """msp_timesum_mfma64 against msp_timesum (the VALU where the one-wave form's
+    waves are not all resident, or n > 256) and numpy, including row, column and
+    time tails and phases up to ~1e6 rad."""
     from muspinsim_amd import _native as N
     rng = np.random.default_rng(100 * n + T)
     E, C, t, w = _timesum_inputs(rng, n, batch, T)
@@ -51,8 +56,8 @@ def test_timesum_mfma64_vs_fp64_valu(gpu_lib, n, T, batch):
     for b in range(batch):
         scale = w[b] * np.abs(C[b]).sum()
         assert np.abs(got[b] - g64[b]).max() <= 1e-13 * scale
-        ph = np.cos(2 * np.pi * (E[b][:, None] - E[b][None, :])[None] * t[:, None, None])
-        ref = w[b] * np.einsum("tij,ij->t", ph, C[b])
+        F = np.exp(2j * np.pi * (E[b] - 0.5 * (E[b][0] + E[b][-1]))[:, None] * t)
+        ref = w[b] * (np.conj(F) * (C[b] @ F)).sum(0).real
         phmax = 2 * np.pi * (E[b].max() - E[b].min()) * t.max()
         assert np.abs(got[b] - ref).max() <= 4e-16 * max(phmax, 1.0) * scale
 
@@ -115,6 +120,22 @@ def test_engine_timesum_paths_vs_oracle(gpu_lib, precision, cfg):
 def test_timesum_one_wave(gpu_lib, n, T, batch, real):
     """msp_timesum's one-wave form, with both kinds of C and of output, a C that
     is neither symmetric nor Hermitian, and every tail of its 16 x 16 x 4 steps."""
+    _check_timesum(gpu_lib, n, T, batch, real)
+
+
+@pytest.mark.parametrize("n,T,batch", [(96, 2250, 11), (97, 2200, 11), (97, 2250, 11),
+                                       (104, 1875, 11), (105, 1855, 11), (105, 1875, 11),
+                                       (113, 1, 1281), (192, 64, 192), (192, 65, 193),
+                                       (256, 720, 11), (256, 740, 11), (257, 33, 11)])
+@pytest.mark.parametrize("real", [0, 1])
+def test_timesum_rule(gpu_lib, n, T, batch, real):
+    """Both sides of the rule between the one-wave and the 64-time form of
+    msp_timesum (n, and waves resident at once), some with 8 instances in the
+    XCD-grouped tile order and the rest in plain order."""
+    _check_timesum(gpu_lib, n, T, batch, real)
+
+
+def _check_timesum(gpu_lib, n, T, batch, real):
     from muspinsim_amd import _native as N
     rng = np.random.default_rng(1000 * n + T + real)
     E, _, t, w = _timesum_inputs(rng, n, batch, T, spread=100.0)
