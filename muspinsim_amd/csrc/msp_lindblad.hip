@@ -6,7 +6,8 @@
 //   k_lindblad_modes  eigendecomposition L = V diag(lambda) V^{-1} (msp_nonsym.h) and
 //                     the mode amplitudes amp_km = (u_k^T V)_m (V^{-1} r)_m; the
 //                     matrix lives in LDS when N <= 64, else in global memory
-//                     (kSplitMinN <= N <= 64 without V: the same steps in three
+//                     (kSplitMinN <= N <= 64 without V, up to N = 20 for batches
+//                     of at most 2048: the same steps in three
 //                     launches, k_lindblad_hess, _schur and _amps)
 //   k_mode_sum        P_k(t) = sum_m amp_km exp(2 pi lambda_m t)
 //   k_mode_integral   I_k = sum_m amp_km / (1/tau - 2 pi lambda_m)
@@ -22,6 +23,8 @@ constexpr int kNT = 256;
 constexpr int kLdsMaxN = 64;    // N at or below this keeps L and Z in LDS
 constexpr int kSplitMinN = 16;  // from here to kLdsMaxN the three-launch form runs without V
 constexpr int kSplitMaxOps = 3; // and up to this many operators
+constexpr int kSplitSmallN = 20;      // up to here only for batches of at most this many:
+constexpr int kSplitSmallBatch = 2048;
 
 __global__ void __launch_bounds__(kNT) k_liouvillian(int n, const double *H, int n_jump,
                                                      const double *Aj, const double *rate,
@@ -171,7 +174,10 @@ __global__ void __launch_bounds__(NT) k_lindblad_modes(int N, double *Lg, const 
 // amps): N = 64 14.5 / 56.9 against 5.1 / 17.4 (2.3 + 14.0 + 0.9), 36 2.6 / 8.5
 // against 1.3 / 4.5, 16 0.62 / 1.03 against 0.37 / 0.99; N = 9 0.23 / 0.36
 // against 0.17 / 0.43, which keeps the one launch.  1024 Liouvillians of a
-// relaxing electron (N = 64): 8.4 against 3.2.
+// relaxing electron (N = 64): 8.4 against 3.2.  Up to N = 20 the one launch holds
+// enough instances per CU to hide its round trips once there are many: N = 17,
+// 2048 matrices 0.76 / 0.76, 4096 1.09 / 1.19; 2048 Liouvillians of N = 16 0.47 /
+// 0.45, 4096 0.67 / 0.71; N = 21, 4096 matrices 2.2 / 1.7.
 
 __device__ inline cdbl lane_c(cdbl v, int l) { return cmk(readlane_f64(v.re, l), readlane_f64(v.im, l)); }
 
@@ -700,7 +706,8 @@ hipError_t launch_lindblad_modes(int N, int batch, double *L, const double *r, i
                                  const double *u, double *lam, double *amp, double *c, double *V,
                                  int32_t *info, double *work, int max_its, hipStream_t s)
 {
-    if (N >= kSplitMinN && N <= kLdsMaxN && !V && n_ops <= kSplitMaxOps) {
+    if (N >= kSplitMinN && N <= kLdsMaxN && !V && n_ops <= kSplitMaxOps &&
+        (N > kSplitSmallN || batch <= kSplitSmallBatch)) {
         ProfScope ps_("k_lindblad_modes", s);
         const size_t lh = sizeof(cdbl) * 64 * (1 + (size_t)n_ops), ls = sizeof(cdbl) * (uh_elems(N) + 64);
         const size_t la = sizeof(cdbl) * ((size_t)N * (N + 1) + 5 * (size_t)N);

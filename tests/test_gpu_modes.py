@@ -82,3 +82,23 @@ def test_eigenvalue_rounding(eng, N):
     err = np.sqrt((((np.sort(lam.imag, 1) - ref) / scale) ** 2).mean())
     assert err <= 2.0 ** -53 * np.sqrt(2 * 2.5 * N)
     assert np.sqrt(((lam.real / scale) ** 2).mean()) <= 2.0 ** -53 * np.sqrt(2 * 2.5 * N)
+
+
+@pytest.mark.parametrize("N", [16, 20, 21])
+@pytest.mark.parametrize("nb", [2048, 2049])
+def test_batch_rule(eng, N, nb):
+    """Both sides of the batch rule up to N = 20: four normal matrices in turn
+    (condition 1), each copy against numpy."""
+    rng = np.random.default_rng(N)
+    G = rng.normal(size=(4, N, N)) + 1j * rng.normal(size=(4, N, N))
+    G = G + np.conj(np.swapaxes(G, 1, 2))
+    r = rng.normal(size=(4, N)) + 1j * rng.normal(size=(4, N))
+    u = rng.normal(size=(4, 2, N)) + 1j * rng.normal(size=(4, 2, N))
+    k = np.arange(nb) % 4
+    lam, amp, _, _ = eng.lindblad_modes(_dev(1j * G[k]), _dev(r[k]), _dev(u[k]))
+    w, V = np.linalg.eigh(G)
+    s = np.abs(w).max()
+    want = np.einsum("bqi,bim,bm,bjm,bj->bq", u, V, np.exp(1j * w / s), V.conj(), r)
+    got = (amp.cpu().numpy() * np.exp(lam.cpu().numpy() / s)[:, None]).sum(2)
+    tol = 1e-15 * N * N * np.linalg.norm(r, axis=1).max() * np.linalg.norm(u, axis=2).max()
+    assert np.abs(got - want[k]).max() <= tol
