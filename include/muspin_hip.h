@@ -234,7 +234,9 @@ int msp_timesum_mixed(int n, int batch, int ntimes, const double *d_E, const dou
  * d_out[b*T + t] = w_b sum_ij C_ij cos(2 pi (E_i - E_j) t), the phases formed
  * exactly as msp_timesum forms them but once per (j, t), the sum over j on
  * FP64 matrix cores.  Agrees with msp_timesum to FP64 rounding.  d_work holds
- * the FP64 phase table (msp_timesum_mfma64_workspace bytes); batch <= 65535. */
+ * the FP64 phase table (msp_timesum_mfma64_workspace bytes, asked for at every n
+ * and not touched where msp_timesum's one-wave kernel runs instead, up to
+ * n = 48); batch <= 65535. */
 size_t msp_timesum_mfma64_workspace(int n, int batch, int ntimes);
 int msp_timesum_mfma64(int n, int batch, int ntimes, const double *d_E, const double *d_C,
                        const double *d_times, const double *d_w, double *d_out, void *d_work,

@@ -26,6 +26,11 @@ MSP_EIGH_JACOBI = 1
 MSP_EIGH_DC = 2
 MSP_EIGH_DC2 = 3
 
+# up to here MSP_EIGH_AUTO and MSP_EIGH_DC are the same kernel, which needs no workspace
+MSP_EIGH_SMALL_N = 16
+# up to here msp_timesum_mfma64 is msp_timesum's kernel (but for a few waves), without a table
+MSP_TIMESUM_WAVE_N = 48
+
 MSP_MAX_SPINS = 16
 MSP_NOALLOC_SCRATCH_BYTES = 64 << 20     # static scratch of msp_eigh_noalloc, per device
 

@@ -7,14 +7,12 @@ dimension n and the number of instances of that dimension, and the best
 choice is measured, not assumed:
 
   eigh          for each bucket n (and a ladder of batch sizes), the LDS
-                Jacobi eigensolver (n <= 64) or Householder + divide and
-                conquer: Jacobi holds one matrix per workgroup for the whole
-                solve, so it wins on latency for small batches and loses on
-                throughput for large ones.
-  timesum       the smallest n from which the mixed-precision time sum
-                (FP32 matrix cores) beats the FP64 one on the same batch, and
-                the smallest n from which the FP64 matrix-core time sum beats
-                the FP64 VALU one.
+                Jacobi eigensolver (n <= 64) or MSP_EIGH_DC (one-wave Jacobi up
+                to n = 16, Householder + divide and conquer above).
+  timesum       the smallest n from which the FP64 time sum from a phase table
+                on matrix cores (msp_timesum_mfma64) beats msp_timesum, and
+                the smallest n from which the mixed-precision time sum (FP32
+                matrix cores) beats the faster FP64 one on the same batch.
   max_chunk     instances per launch of the n = 192 divide-and-conquer path.
 
 `tune()` times them with HIP events around the library calls and returns a
@@ -34,7 +32,7 @@ DEFAULT_PATH = os.path.join(HERE, "tuning.json")
 
 EIGH_NS = (4, 8, 12, 16, 24, 32, 48, 64)
 EIGH_BATCHES = (64, 256, 1024, 4096, 16384)
-TIMESUM_NS = (16, 24, 32, 48, 64, 96, 128)
+TIMESUM_NS = (16, 24, 32, 40, 48, 64, 72, 80, 96, 112, 128, 192, 256)
 
 
 def _events_ms(fn, reps):
@@ -119,39 +117,13 @@ def tune_eigh(lib, ns=EIGH_NS, batches=EIGH_BATCHES, reps=3):
     return eigh_ladders(raw), raw
 
 
-def tune_timesum(lib, ns=TIMESUM_NS, ntimes=2000, batch=256, reps=3):
-    """Smallest n (of ns) from which the mixed-precision time sum is faster
-    than the FP64 one, and the raw timings."""
-    import torch
-    from . import _native as N
-    raw = {}
-    first = None
-    st = torch.cuda.current_stream().cuda_stream
-    t = torch.linspace(0, 10, ntimes, dtype=torch.float64, device="cuda")
-    for n in ns:
-        E = torch.sort(torch.randn((batch, n), dtype=torch.float64, device="cuda") * 50, dim=1).values
-        C = torch.randn((batch, n, n), dtype=torch.float64, device="cuda")
-        C = ((C + C.transpose(1, 2)) / 2).contiguous()
-        out = torch.empty((batch, ntimes), dtype=torch.float64, device="cuda")
-        ws = lib.msp_timesum_mixed_workspace(n, batch, ntimes)
-        work = torch.empty((max(ws, 8) // 8,), dtype=torch.float64, device="cuda")
-        t64 = _events_ms(lambda: N.check(lib.msp_timesum(n, batch, ntimes, E.data_ptr(), C.data_ptr(),
-                                                         1, t.data_ptr(), None, 0, out.data_ptr(),
-                                                         st)), reps)
-        t32 = _events_ms(lambda: N.check(lib.msp_timesum_mixed(n, batch, ntimes, E.data_ptr(),
-                                                               C.data_ptr(), t.data_ptr(), None,
-                                                               out.data_ptr(), work.data_ptr(), ws,
-                                                               st)), reps)
-        raw[str(n)] = {"fp64_ms": t64, "mixed_ms": t32}
-        if first is None and t32 < t64:
-            first = n
-    return (first if first is not None else 1 << 30), raw
-
-
-def tune_timesum64(lib, ns=TIMESUM_NS + (192, 256), ntimes=2000, batch=256, reps=3, tol=0.05):
-    """Smallest n (of ns) from which the FP64 matrix-core time sum (phase
-    table + MFMA GEMM) is faster than the FP64 VALU one by more than `tol`
-    at this n and every larger n measured, and the raw timings."""
+def tune_timesum(lib, ns=TIMESUM_NS, ntimes=2000, batch=256, reps=3, tol=0.05):
+    """(first_table, first_mixed, raw): the smallest n (of ns) where
+    msp_timesum_mfma64 is faster than msp_timesum and from which on it is never
+    slower by more than `tol`, the same for the mixed-precision time sum against
+    the faster of the two, and the timings of all three.  Up to
+    n = MSP_TIMESUM_WAVE_N the first two are one kernel; only msp_timesum is
+    timed there, which needs no phase table."""
     import torch
     from . import _native as N
     raw = {}
@@ -162,33 +134,43 @@ def tune_timesum64(lib, ns=TIMESUM_NS + (192, 256), ntimes=2000, batch=256, reps
         C = torch.randn((batch, n, n), dtype=torch.float64, device="cuda")
         C = ((C + C.transpose(1, 2)) / 2).contiguous()
         out = torch.empty((batch, ntimes), dtype=torch.float64, device="cuda")
-        ws = lib.msp_timesum_mfma64_workspace(n, batch, ntimes)
-        work = torch.empty((max(ws, 8) // 8,), dtype=torch.float64, device="cuda")
-        t64 = _events_ms(lambda: N.check(lib.msp_timesum(n, batch, ntimes, E.data_ptr(), C.data_ptr(),
-                                                         1, t.data_ptr(), None, 0, out.data_ptr(),
-                                                         st)), reps)
-        tm = _events_ms(lambda: N.check(lib.msp_timesum_mfma64(n, batch, ntimes, E.data_ptr(),
-                                                               C.data_ptr(), t.data_ptr(), None,
-                                                               out.data_ptr(), work.data_ptr(), ws,
-                                                               st)), reps)
-        raw[str(n)] = {"valu_ms": t64, "mfma_ms": tm}
-        del E, C, out, work
+
+        def table_ms(fn, workspace):
+            ws = workspace(n, batch, ntimes)
+            work = torch.empty((max(ws, 8) // 8,), dtype=torch.float64, device="cuda")
+            return _events_ms(lambda: N.check(fn(n, batch, ntimes, E.data_ptr(), C.data_ptr(),
+                                                 t.data_ptr(), None, out.data_ptr(),
+                                                 work.data_ptr(), ws, st)), reps)
+
+        r = {"direct_ms": _events_ms(lambda: N.check(lib.msp_timesum(
+            n, batch, ntimes, E.data_ptr(), C.data_ptr(), 1, t.data_ptr(), None, 0,
+            out.data_ptr(), st)), reps)}
+        if n > N.MSP_TIMESUM_WAVE_N:
+            r["table_ms"] = table_ms(lib.msp_timesum_mfma64, lib.msp_timesum_mfma64_workspace)
+        r["mixed_ms"] = table_ms(lib.msp_timesum_mixed, lib.msp_timesum_mixed_workspace)
+        raw[str(n)] = r
+        del E, C, out
         torch.cuda.empty_cache()
-    return timesum64_threshold(raw, tol), raw
+    return timesum_thresholds(raw, tol) + (raw,)
 
 
-def timesum64_threshold(raw, tol=0.05):
-    """The smallest n from which every measured n has the matrix-core time
-    sum faster by more than `tol` (a very large n when none does)."""
-    ns = sorted(int(k) for k in raw)
-    first = 1 << 30
-    for n in reversed(ns):
-        r = raw[str(n)]
-        if r["mfma_ms"] < r["valu_ms"] * (1.0 - tol):
-            first = n
-        else:
-            break
-    return first
+def timesum_thresholds(raw, tol=0.05):
+    """(first_table, first_mixed) from timings {"<n>": {"direct_ms", "table_ms"
+    (absent where it is the same kernel), "mixed_ms"}}; a very large n when there
+    is none."""
+    def first(pair):
+        best = 1 << 30
+        for n in sorted((int(k) for k in raw), reverse=True):
+            new, old = pair(raw[str(n)])
+            if new > old * (1.0 + tol):
+                break
+            if new < old:
+                best = n
+        return best
+
+    never = float("inf")
+    return (first(lambda r: (r.get("table_ms", never), r["direct_ms"])),
+            first(lambda r: (r["mixed_ms"], min(r.get("table_ms", never), r["direct_ms"]))))
 
 
 def tune_chunk(candidates=(2048, 4096, 8192), nfields=40, nori=500):
@@ -227,17 +209,15 @@ def tune(quick=False):
     reps = 2 if quick else 3
     batches = (64, 1024, 8192) if quick else EIGH_BATCHES
     eigh, eigh_raw = tune_eigh(lib, batches=batches, reps=reps)
-    ts_min, ts_raw = tune_timesum(lib, reps=reps)
-    ts64_min, ts64_raw = tune_timesum64(lib, reps=reps)
+    table_min, mixed_min, ts_raw = tune_timesum(lib, reps=reps)
     chunk, chunk_raw = tune_chunk() if not quick else (8192, {})
     return {
         "device": torch.cuda.get_device_properties(0).gcnArchName,
         "eigh": eigh,
-        "mixed_timesum_min_n": ts_min,
-        "fp64_timesum_mfma_min_n": ts64_min,
+        "mixed_timesum_min_n": mixed_min,
+        "fp64_timesum_mfma_min_n": table_min,
         "max_chunk": chunk,
-        "measured": {"eigh_ms": eigh_raw, "timesum_ms": ts_raw, "timesum64_ms": ts64_raw,
-                     "chunk_ms": chunk_raw},
+        "measured": {"eigh_ms": eigh_raw, "timesum_ms": ts_raw, "chunk_ms": chunk_raw},
     }
 
 

@@ -92,3 +92,30 @@ def test_autotune_ladder_hysteresis():
     assert t["12"] == [[1, "jacobi"]]
     assert t["16"] == [[1, "dc"], [1024, "jacobi"]]
     assert autotune.eigh_ladders(raw, tol=0.0)["12"] == [[1, "jacobi"], [256, "dc"], [1024, "jacobi"]]
+
+
+def test_timesum_thresholds():
+    """First n where a time sum is faster and from which it is never slower by
+    more than tol; sizes without a phase-table timing (the same kernel) never
+    select the table."""
+    from muspinsim_amd import autotune
+    raw = {"16": {"direct_ms": 1.0, "mixed_ms": 0.5}, "48": {"direct_ms": 4.0, "mixed_ms": 4.5},
+           "64": {"direct_ms": 8.0, "table_ms": 7.0, "mixed_ms": 6.0},
+           "72": {"direct_ms": 9.0, "table_ms": 9.9, "mixed_ms": 9.1},
+           "96": {"direct_ms": 20.0, "table_ms": 15.0, "mixed_ms": 13.0}}
+    assert autotune.timesum_thresholds(raw, 0.05) == (96, 64)
+    assert autotune.timesum_thresholds(raw, 0.15) == (64, 16)
+    assert autotune.timesum_thresholds(raw, 0.0) == (96, 96)
+    raw["96"].update(table_ms=30.0, mixed_ms=30.0)
+    assert autotune.timesum_thresholds(raw) == (1 << 30, 1 << 30)
+
+
+def test_no_phase_table_where_the_time_sum_needs_none():
+    """Up to n = 48 msp_timesum and msp_timesum_mfma64 run one kernel: the shipped
+    tuning does not make plans allocate the phase table there."""
+    from muspinsim_amd import _native as N
+    from muspinsim_amd import autotune
+    t = autotune.load()
+    assert t["fp64_timesum_mfma_min_n"] > N.MSP_TIMESUM_WAVE_N
+    assert all("table_ms" not in r for n, r in t["measured"]["timesum_ms"].items()
+               if int(n) <= N.MSP_TIMESUM_WAVE_N)
