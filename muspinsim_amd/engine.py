@@ -125,8 +125,8 @@ class SpinEngine:
     """Runs instance batches through the HIP pipeline on one device."""
 
     # A chunk's buffers take up to 32 GiB of the 288 GiB of HBM: at n = 192
-    # that is 8192 instances, 16 full residency waves of the two-per-CU
-    # tridiagonalisation, so partial last waves and launch gaps are rare.
+    # that is 8192 instances, 32 full residency waves of the tridiagonalisation
+    # (one workgroup per CU), so partial last waves and launch gaps are rare.
     # precision "fp64": every stage in FP64 (the drop-in, max|dP| <= 1e-10
     # against the FP64 oracle); "mixed": the time sums of the real routes run
     # on FP32 matrix cores with FP64 phase reduction and FP64 sums over rows
@@ -213,6 +213,9 @@ class SpinEngine:
             # msp_eigh's own choice here is the LDS Jacobi kernel, which needs
             # no workspace; with one, divide and conquer is faster
             m = N.MSP_EIGH_DC
+        if m == N.MSP_EIGH_DC and n <= N.MSP_EIGH_SMALL_N:
+            # the same kernel by the name that asks for no workspace
+            m = N.MSP_EIGH_AUTO
         return m
 
     def per_instance_bytes(self, n, complex_rho, method=None):
@@ -228,10 +231,11 @@ class SpinEngine:
     # ---------------------------------------------------------------- stages
     def _dc_lower(self, n, method=None):
         """Whether msp_eigh with this method reads only the lower triangle of
-        an n x n input (the D&C path up to n = 1024)."""
+        an n x n input (the one-wave kernel up to n = 16 and the D&C path up to
+        n = 1024)."""
         m = self.method if method is None else method
         if m == N.MSP_EIGH_AUTO:
-            m = N.MSP_EIGH_JACOBI if n <= 64 else N.MSP_EIGH_DC
+            m = N.MSP_EIGH_JACOBI if N.MSP_EIGH_SMALL_N < n <= 64 else N.MSP_EIGH_DC
         return m == N.MSP_EIGH_DC and n <= 1024
 
     def eigh(self, H, method=None):
@@ -565,7 +569,7 @@ class SpinEngine:
 
             N.check(L.msp_rotate_fields(nb, p(g.q), p(g.B), p(g.Bint), p(g.p),
                                         g.Br.data_ptr(), g.pr.data_ptr(), st))
-            # the D&C eigensolver (n <= 1024) reads the lower triangle only
+            # these eigensolvers read the lower triangle only
             build = (L.msp_build_h_lower if g.route != "lindblad" and self._dc_lower(n, g.method)
                      else L.msp_build_h)
             if g.base is not None:

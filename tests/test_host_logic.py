@@ -119,3 +119,24 @@ def test_no_phase_table_where_the_time_sum_needs_none():
     assert t["fp64_timesum_mfma_min_n"] > N.MSP_TIMESUM_WAVE_N
     assert all("table_ms" not in r for n, r in t["measured"]["timesum_ms"].items()
                if int(n) <= N.MSP_TIMESUM_WAVE_N)
+
+
+def test_small_eigenproblems_take_no_workspace():
+    """n <= 16: whatever the tuned choice, a plan's eigensolver asks for no
+    workspace unless the caller named the method; the lower triangle suffices."""
+    from muspinsim_amd import _native as N
+    from muspinsim_amd import autotune
+    from muspinsim_amd.engine import SpinEngine
+    eng = object.__new__(SpinEngine)
+    lib = N.load_library()
+    for tuning in (None, autotune.load()):
+        eng.tuning, eng.method = tuning, N.MSP_EIGH_AUTO
+        for n in (2, 4, 6, 8, 12, 16):
+            m = eng.method_for(n, 1000)
+            assert lib.msp_eigh_workspace(n, 1000, m) == 0
+            assert eng._dc_lower(n, m)
+            assert eng.per_instance_bytes(n, False, m) == 4 * n * n * 16 + n * 32
+        assert eng.method_for(18, 1000) == N.MSP_EIGH_DC and eng._dc_lower(18, N.MSP_EIGH_DC)
+        assert not eng._dc_lower(18, N.MSP_EIGH_AUTO)
+    eng.method = N.MSP_EIGH_DC
+    assert eng.method_for(16, 10) == N.MSP_EIGH_DC
