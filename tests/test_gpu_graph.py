@@ -18,10 +18,12 @@ def _herm(rng, n):
     return (X + X.conj().T) / 2
 
 
-def test_capi_graph_replays_eigh(gpu_lib):
+@pytest.mark.parametrize("n,B", [(16, 9), (192, 6), (320, 2)])
+def test_capi_graph_replays_eigh(gpu_lib, n, B):
+    """One-wave Jacobi, the register-resident reduction and the one spread over
+    many launches (2 n - 1 graph nodes)."""
     from muspinsim_amd import _native as N
     L = N.lib()
-    n, B = 192, 6
     rng = np.random.default_rng(3)
     H0 = torch.as_tensor(np.array([_herm(rng, n) for _ in range(B)])).cuda()
     H = torch.empty_like(H0)

@@ -1,7 +1,7 @@
 """Hermitian eigensolver at the edges of its kernels: the one-wave Jacobi kernel
-(n <= 16) and, through the divide and conquer, the register-resident Householder
-tridiagonalisation (n <= 256), on structured matrices and on both sides of its
-batch rule."""
+(n <= 16) and, through the divide and conquer, the Householder tridiagonalisations
+(register-resident n <= 256, spread over many workgroups and panels above), on
+structured matrices and on both sides of each batch rule."""
 
 import numpy as np
 import pytest
@@ -30,8 +30,12 @@ def _check(eng, Hs, method=None):
     low[:, np.triu_indices(n, 1)[0], np.triu_indices(n, 1)[1]] = np.nan
     E, U, info = eng.eigh(torch.as_tensor(low).cuda(),
                           method=N.MSP_EIGH_DC if method is None else method)
-    E, U = E.cpu().numpy(), U.cpu().numpy()
     assert np.all(info.cpu().numpy() == 0)
+    _accurate(Hs, E.cpu().numpy(), U.cpu().numpy())
+
+
+def _accurate(Hs, E, U):
+    n = Hs.shape[1]
     nrm = np.maximum(np.abs(E).max(1), 1e-300)
     assert np.all(np.abs(E - np.linalg.eigvalsh(Hs)).max(1) <= 1e-14 * n * nrm)
     assert np.all(np.abs(Hs @ U - U * E[:, None, :]).max((1, 2)) <= 1e-14 * n * nrm)
@@ -118,3 +122,41 @@ def test_small_norms(eng, n, sweeps):
     U = U.cpu().numpy()
     off = (U.real.astype(np.longdouble) ** 2 + U.imag.astype(np.longdouble) ** 2).sum(1) - 1
     assert np.sqrt(float((off ** 2).mean())) <= 1.4 * 2.0 ** -53 * np.sqrt(sweeps * (n - 1))
+
+
+@pytest.mark.parametrize("n,batch", [(257, 32), (257, 33), (512, 96), (512, 97), (513, 96), (513, 97),
+                                     (1023, 193), (1024, 192), (1024, 193)])
+def test_large_batch_rule(eng, n, batch):
+    """Both sides of the line between the spread reduction (batch <= 192 and 4
+    batch <= n - 128) and the panel kernel (panels in LDS up to n = 512, in the
+    workspace above): three matrices in turn, checked once, every copy alike."""
+    from muspinsim_amd import _native as N
+    rng = np.random.default_rng(n)
+    H = np.array([_herm(rng, n) for _ in range(2)] + [np.diag(rng.normal(size=n)) + 0j])
+    k = torch.arange(batch, device="cuda") % 3
+    low = np.where(np.tri(n, dtype=bool), H, np.nan)
+    E, U, info = eng.eigh(torch.as_tensor(low).cuda()[k], method=N.MSP_EIGH_DC)
+    assert int(info.abs().max()) == 0
+    assert torch.equal(E, E[:3][k])
+    for b in range(3, batch):
+        assert torch.equal(U[b], U[b % 3])
+    _accurate(H, E[:3].cpu().numpy(), U[:3].cpu().numpy())
+
+
+def test_large_on_two_streams(eng):
+    """Two spread reductions side by side on two streams, each with its own
+    workspace, as dimension groups of one plan run them."""
+    from muspinsim_amd import _native as N
+    rng = np.random.default_rng(5)
+    Hs = [torch.as_tensor(np.array([_herm(rng, n) for _ in range(4)])).cuda() for n in (300, 420)]
+    alone = [eng.eigh(H.clone(), method=N.MSP_EIGH_DC) for H in Hs]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in Hs]
+    for _ in range(3):
+        out = []
+        for s, H in zip(streams, Hs):
+            with torch.cuda.stream(s):
+                out.append(eng.eigh(H.clone(), method=N.MSP_EIGH_DC))
+        torch.cuda.synchronize()
+        for (E, U, _), (E0, U0, _) in zip(out, alone):
+            assert torch.equal(E, E0) and torch.equal(U, U0)
