@@ -1,5 +1,5 @@
 // Panel-blocked Householder tridiagonalisation that reads and writes only the
-// lower triangle (gfx950, one workgroup of W = 4 or 8 waves per matrix).
+// lower triangle (gfx950, one workgroup of W = 8 waves per matrix, n > 256).
 //
 // Same reduction as tridiag_team in msp_tridiag.h (A = Q T Q^H, reflector
 // tails stored below the subdiagonal, d/e/tau out), organised for HBM:
@@ -21,11 +21,8 @@ namespace {
 
 constexpr int kCpRows = 4;      // LDS rows of per-wave column partials
 constexpr int kPanelRows = 8;   // rows per batched pass of the end-of-panel update
-#ifndef MSP_TD_RB
-#define MSP_TD_RB 4     // rows per batched pass of the A22 v product (64-lane rows)
-#endif
 #ifndef MSP_TD_WL
-#define MSP_TD_WL 8     // waves per workgroup above n = 192
+#define MSP_TD_WL 8     // waves per workgroup
 #endif
 #ifndef MSP_TD_RBMAX
 #define MSP_TD_RBMAX 4  // most rows in one pass of the 64-lane-row A22 v product
@@ -44,22 +41,20 @@ constexpr int kPanelRows = 8;   // rows per batched pass of the end-of-panel upd
 __device__ inline double wave_sum(double v) { return wave_sum_all(v); }
 
 // Column partials of one step, every thread of the workgroup calling: wave w
-// stores its per-lane sums acc[q] (column c0 + CS q, lanes with `writer`) in
-// LDS row w % 4 of cp; with W = 8 the waves w and w + 4 share a row, the
-// second adding to the first after a barrier, so the order of the sum is
-// fixed.  (The caller's barrier ends the last phase.)
-template <int W, int Q, int CS>
-__device__ inline void store_colpart(int n, int c0, int wave, bool writer, const cdbl (&acc)[Q],
-                                     cdbl *cp)
+// stores its per-lane sums acc[q] (column c0 + 64 q) in LDS row w % 4 of cp; the
+// waves w and w + 4 share a row, the second adding to the first after a barrier,
+// so the order of the sum is fixed.  (The caller's barrier ends the last phase.)
+template <int W, int Q>
+__device__ inline void store_colpart(int n, int c0, int wave, const cdbl (&acc)[Q], cdbl *cp)
 {
     static_assert(W % kCpRows == 0, "W is a multiple of the partial rows");
     for (int ph = 0; ph < W / kCpRows; ++ph) {
         if (ph > 0) __syncthreads();
-        if (wave / kCpRows == ph && writer) {
+        if (wave / kCpRows == ph) {
             cdbl *row = cp + (size_t)(wave % kCpRows) * n;
 #pragma unroll
             for (int q = 0; q < Q; ++q) {
-                const int c = c0 + CS * q;
+                const int c = c0 + 64 * q;
                 if (c < n) row[c] = (ph > 0) ? cadd(row[c], acc[q]) : acc[q];
             }
         }
@@ -248,7 +243,7 @@ __device__ __forceinline__ int a22v_rows(int n, int k, int i0, int lane, const c
 template <int W, int NB, int QMAX, int RB, bool GP>
 __global__ void __launch_bounds__(64 * W) k_tridiag_lp(int n, double *H, double *E, double *work)
 {
-    static_assert(W == 4 || W == 8, "4 or 8 waves per matrix");
+    static_assert(W == 8, "the column partials take 8 waves in two phases");
     constexpr int kThreads = 64 * W;
     extern __shared__ __align__(16) unsigned char smem[];
     const int b = blockIdx.x;
@@ -363,7 +358,7 @@ __global__ void __launch_bounds__(64 * W) k_tridiag_lp(int n, double *H, double 
                 // lane and row: neither loaded nor used)
                 for (int i0 = k + 1 + wave; i0 < n;)
                     i0 += a22v_rows<W, QMAX, RB>(n, k, i0, lane, A, vb, pb, nxt, colacc);
-                store_colpart<W, QMAX, 64>(n, k + 1 + lane, wave, true, colacc, cp);
+                store_colpart<W, QMAX>(n, k + 1 + lane, wave, colacc, cp);
                 __syncthreads();
                 // (e) p = tau (A22 v - Vp y1 - Wp y2), and p^H v
                 double pre = 0.0, pim = 0.0;

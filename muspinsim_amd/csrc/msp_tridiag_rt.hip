@@ -121,7 +121,7 @@ struct RtShape {
     // LDS: x', column k + 1, v and w, column sums per wave, row sums per lane,
     // scale, tau scale, -|tau scale|^2 / 2, and a share of v^H A22 v per wave
     static constexpr int CDBL = 4 * NP + W * NP + 64 * W * NS + 3;
-    static constexpr size_t LDS = sizeof(cdbl) * CDBL + sizeof(double) * ((W + 1) & ~1);
+    static constexpr size_t LDS = sizeof(cdbl) * CDBL + sizeof(double) * W;
 };
 
 template <int W, int NS, int OCC, int JC>
@@ -129,7 +129,7 @@ __global__ void __launch_bounds__(64 * W, OCC) k_tridiag_rt(int n, double *H, do
 {
     using T = RtShape<W, NS, JC>;
     constexpr int SR = T::SR, NJ = T::NJ, NC = T::NC, NP = T::NP;
-    static_assert(NS <= 8, "two lanes per row of a wave");
+    static_assert(NS <= 8 && W % 2 == 0, "two lanes per row of a wave, each on half the waves' sums");
     static_assert(JC == 0 || W == 8, "a strip's diagonal region is one pair of blocks");
     extern __shared__ __align__(16) unsigned char smem[];
     cdbl *col = (cdbl *)smem;                  // x': zero up to row k
@@ -468,8 +468,7 @@ __global__ void __launch_bounds__(64 * W, OCC) k_tridiag_rt(int n, double *H, do
 #pragma unroll
             for (int w = 0; w < W; ++w) rho += dot[w];
 #pragma unroll
-            for (int w = 0; w < (W + 1) / 2; ++w)
-                if (W > 1 || h == 0) y = cadd(y, P[(w + h * (W / 2)) * NP + i]);
+            for (int w = 0; w < W / 2; ++w) y = cadd(y, P[(w + h * (W / 2)) * NP + i]);
             double t = y.re;
             swap32(y.re, t);
             y.re += t;
@@ -501,8 +500,8 @@ hipError_t rt_launch(int n, int batch, double *H, double *E, double *work, hipSt
 
 }  // namespace
 
-// Waves and strips by n (n <= 16 has an eigensolver of its own): few waves for small matrices, so that many
-// matrices share a CU, four waves where two or more workgroups still fit its
+// Waves and strips by n (n <= 16 has an eigensolver of its own): few waves for
+// small matrices, so that many matrices share a CU, four waves where two or more workgroups still fit its
 // registers (n <= 128), eight above.  Strips of 4 W rows cover n closely: a
 // strip too many costs 10 to 20 %.
 // Up to 512 matrices run at most two to a CU and take the form with the
