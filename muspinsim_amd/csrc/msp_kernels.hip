@@ -189,7 +189,7 @@ __global__ void __launch_bounds__(256) k_build_h(int n, const MspSystem *systems
     ((cdbl *)H)[(size_t)b * n * n + idx] = h_element(n, systems[s], terms, bm, Br + 3 * b, zeeman, idx);
 }
 
-// The same for large n, ept elements per thread.  With the digits packed in LDS,
+// The same for small and large n, ept elements per thread.  With the digits packed in LDS,
 // one XOR tells an element whose row and column differ in three spins or more
 // (zero, or the base: all but a few per row of a large system) and which spins
 // differ in the others; systems with a multiplicity above 16 take the
@@ -1078,12 +1078,17 @@ hipError_t launch_build_h(int n, int batch, const MspSystem *systems, const MspT
     // A thread of the packed form takes up to 16 elements, sharing one digit
     // table, while 8192 workgroups are left.  It pays from about four on and
     // above n = 256; with fewer elements the slowest wave's term loop decides, or
-    // too few elements are skipped.  us an element per thread / packed, lower
-    // triangles: n = 288, 80 matrices 365 / 380, 300 1295 / 900; n = 2048, one 365
-    // / 385, six 2300 / 1460; n = 256, 300 2340 / 2560
+    // too few elements are skipped.  It also pays for small n, which one workgroup
+    // covers (never with a multiplicity above 16), unless so many hardly filled
+    // workgroups wait for their table.  us an element per thread /
+    // packed, lower triangles: n = 288, 80 matrices 365 / 380, 300 1295 / 900; n =
+    // 2048, one 365 / 385, six 2300 / 1460; n = 256, 300 2340 / 2560; n = 64, 20 53 /
+    // 73; n = 16, one 11.5 / 9.8, 5000 88 / 75; n = 8, 1200 5.9 / 5.2, 20000 34.7 /
+    // 38.5
     const size_t wgs = cdiv((size_t)n * n, 256);
-    if (n > 256 && wgs * batch >= 4 * 8192) {
-        const int ept = (int)std::min<size_t>(16, wgs * batch / 8192);
+    if ((n > 8 && n <= 16) || (n > 4 && n <= 8 && batch <= 1024) ||
+        (n > 256 && wgs * batch >= 4 * 8192)) {
+        const int ept = (int)std::min<size_t>(16, std::max<size_t>(1, wgs * batch / 8192));
         hipLaunchKernelGGL(k_build_h_packed, dim3(cdiv(wgs, ept), batch), dim3(256),
                            sizeof(unsigned long long) * n, s, n, systems, terms, sys_id, Br, base,
                            zeeman, lower, ept, H);
