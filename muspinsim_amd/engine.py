@@ -161,7 +161,7 @@ class SpinEngine:
         self.mixed_min_n = int(t.get("mixed_timesum_min_n", 48))
         self.mixed_min_work = float(t.get("mixed_timesum_min_work", 1e9))
         # FP64 time sum from a phase table (plain precision) from this n on
-        self.mfma64_min_n = int(t.get("fp64_timesum_mfma_min_n", 96))
+        self.mfma64_min_n = int(t.get("fp64_timesum_mfma_min_n", 64))
         self.precision = precision
         self.group_streams = int(group_streams)
         self.chunk_bytes = chunk_bytes
@@ -468,7 +468,7 @@ class SpinEngine:
         g.tswork, g.tswsb, g.tsmode = None, 0, None
         # The real routes' time sum runs on matrix cores from a phase table:
         # FP32 products for precision="mixed", FP64 for "fp64".  Below the
-        # tuned dimension (48 and 96 without tuning) msp_timesum, which needs no
+        # tuned dimension (48 and 64 without tuning) msp_timesum, which needs no
         # table, is faster, and below about 1e9 multiply-adds per launch the
         # phase-table launch is not repaid either (few instances, short time
         # axes).
