@@ -25,7 +25,7 @@
 // What bounds it: at n = 192 about 480 vector instructions per wave and column
 // (300 of them FP64 FMAs, 190 of those the live lower triangle's) keep the
 // SIMDs half busy; the rest is the reflector's serial chain, the barriers and
-// LDS (37 % busy).  At one 8-wave workgroup per CU nothing covers the barriers;
+// LDS (43 % busy, a fifth of it bank conflicts).  At one 8-wave workgroup per CU nothing covers the barriers;
 // below n = 128 two to sixteen workgroups share a CU.
 // The panel kernel re-reads the trailing triangle once per column (at n = 192
 // 5.2 TB/s past L2); here the matrix is read once.  ms per 4096 matrices, panel
