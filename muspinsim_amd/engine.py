@@ -209,9 +209,11 @@ class SpinEngine:
         m = autotune.eigh_method(self.tuning, n, count)
         if m == N.MSP_EIGH_JACOBI and n > 64:
             m = N.MSP_EIGH_AUTO
-        if m == N.MSP_EIGH_AUTO and 16 < n <= 64:
+        if m == N.MSP_EIGH_AUTO and 16 < n <= 64 and (n > 18 or count < 2048):
             # msp_eigh's own choice here is the LDS Jacobi kernel, which needs
-            # no workspace; with one, divide and conquer is faster
+            # no workspace; with one, divide and conquer is faster (ms Jacobi /
+            # DC, n = 18: 256 matrices 0.20 / 0.15, 2048 0.37 / 0.39, 16384 2.45 /
+            # 2.66; n = 20: 2048 0.46 / 0.40, 16384 3.1 / 2.8)
             m = N.MSP_EIGH_DC
         if m == N.MSP_EIGH_DC and n <= N.MSP_EIGH_SMALL_N:
             # the same kernel by the name that asks for no workspace

@@ -138,5 +138,9 @@ def test_small_eigenproblems_take_no_workspace():
             assert eng.per_instance_bytes(n, False, m) == 4 * n * n * 16 + n * 32
         assert eng.method_for(18, 1000) == N.MSP_EIGH_DC and eng._dc_lower(18, N.MSP_EIGH_DC)
         assert not eng._dc_lower(18, N.MSP_EIGH_AUTO)
+        # many matrices of n = 18 stay with the LDS Jacobi kernel
+        assert eng.method_for(18, 2047) == N.MSP_EIGH_DC
+        assert eng.method_for(18, 2048) == N.MSP_EIGH_AUTO
+        assert eng.method_for(20, 1 << 20) == N.MSP_EIGH_DC
     eng.method = N.MSP_EIGH_DC
     assert eng.method_for(16, 10) == N.MSP_EIGH_DC
