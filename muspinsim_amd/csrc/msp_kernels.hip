@@ -1075,19 +1075,27 @@ hipError_t launch_build_h(int n, int batch, const MspSystem *systems, const MspT
                            Br, base, lower, H);
         return hipGetLastError();
     }
-    // A thread of the packed form takes up to 16 elements, sharing one digit
-    // table, while 8192 workgroups are left.  It pays from about four on and
-    // above n = 256; with fewer elements the slowest wave's term loop decides, or
-    // too few elements are skipped.  It also pays for small n, which one workgroup
-    // covers (never with a multiplicity above 16), unless so many hardly filled
-    // workgroups wait for their table.  us an element per thread /
-    // packed, lower triangles: n = 288, 80 matrices 365 / 380, 300 1295 / 900; n =
-    // 2048, one 365 / 385, six 2300 / 1460; n = 256, 300 2340 / 2560; n = 64, 20 53 /
-    // 73; n = 16, one 11.5 / 9.8, 5000 88 / 75; n = 8, 1200 5.9 / 5.2, 20000 34.7 /
-    // 38.5
+    // The packed form, by size (us an element per thread / packed, lower
+    // triangles):
+    //   n <= 4: too few elements to share a table (20000 matrices of n = 4 33 / 38);
+    //   n <= 8: up to 1024 matrices (1200 of n = 8 5.9 / 5.2, 20000 34.7 / 38.5);
+    //   n <= 30: always, four spins at most (one matrix of n = 16 11.3 / 9.9, of 24
+    //   14.6 / 13.3; 5000 of n = 24 200 / 174);
+    //   n <= 32: from 1024 matrices (5 spins: 20 27 / 29, 1200 126 / 118); digits
+    //   always pack up to here but for a lone spin;
+    //   n <= 256: no, with five spins and more the slowest wave's term loop decides
+    //   (n = 64, 20 53 / 73; n = 256, 300 2340 / 2560);
+    //   above, where most elements are skipped, once a thread takes four elements or
+    //   more with 8192 workgroups left (n = 288, 80 365 / 380, 300 1295 / 900; n =
+    //   2048, one 365 / 385, six 2300 / 1460).
     const size_t wgs = cdiv((size_t)n * n, 256);
-    if ((n > 8 && n <= 16) || (n > 4 && n <= 8 && batch <= 1024) ||
-        (n > 256 && wgs * batch >= 4 * 8192)) {
+    const bool packed = n <= 4     ? false
+                        : n <= 8   ? batch <= 1024
+                        : n <= 30  ? true
+                        : n <= 32  ? batch >= 1024
+                        : n <= 256 ? false
+                                   : wgs * batch >= 4 * 8192;
+    if (packed) {
         const int ept = (int)std::min<size_t>(16, std::max<size_t>(1, wgs * batch / 8192));
         hipLaunchKernelGGL(k_build_h_packed, dim3(cdiv(wgs, ept), batch), dim3(256),
                            sizeof(unsigned long long) * n, s, n, systems, terms, sys_id, Br, base,

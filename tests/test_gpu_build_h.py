@@ -1,6 +1,6 @@
 """Hamiltonian build from the terms against the oracle: an element per thread, and
-with packed spin digits one (4 < n <= 16) or several (n > 256 and many elements),
-on both sides of each rule, digits up to the packed limit of 15 and above it, full
+with packed spin digits one or several (4 < n <= 32, and n > 256 with many
+elements), on both sides of each rule, digits up to the packed limit of 15 and above it, full
 matrices and lower triangles."""
 
 import numpy as np
@@ -14,7 +14,9 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("lower", [False, True])
 @pytest.mark.parametrize("Is,nb", [([0.5], 1), ([0.5, 0.5], 3), ([2.0], 3), ([7.5], 3), ([8.0], 3),
-                                   ([0.5, 1.5], 1024), ([0.5, 1.5], 1025),
+                                   ([0.5, 1.5], 1024), ([0.5, 1.5], 1025), ([0.5, 0.5, 1.0, 0.5], 9),
+                                   ([0.5, 7.0], 9000), ([0.5] * 5, 1023), ([0.5] * 5, 1024),
+                                   ([0.5, 8.0], 1030),
                                    ([0.5, 0.5, 1.5], 9000), ([0.5, 1.0, 0.5], 5000), ([0.5] * 8, 3),
                                    ([0.5] * 8, 40), ([0.5, 3.5, 0.5, 1.0], 70), ([7.5, 0.5], 600),
                                    ([0.5, 8.5], 600),
