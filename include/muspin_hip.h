@@ -129,7 +129,8 @@ int msp_build_h_lower(int n, int batch, const MspSystem *d_systems, const MspTer
 
 /* Batched Hermitian eigendecomposition.  d_H is destroyed.  d_E: batch x n
  * ascending eigenvalues; d_U: batch x n x n eigenvectors (columns).
- * d_info: batch int32, 0 = converged. */
+ * d_info: batch int32, 0 = converged; up to n = 16 by MSP_EIGH_AUTO or _DC a
+ * matrix with a NaN or infinite entry gives 1 and NaN results. */
 size_t msp_eigh_workspace(int n, int batch, int method);
 int msp_eigh(int n, int batch, double *d_H, double *d_E, double *d_U, int32_t *d_info,
              int method, void *d_work, size_t work_bytes, void *stream);
